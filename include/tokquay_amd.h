@@ -16,6 +16,7 @@
  * plus two kernels of the model step around them:
  *
  *   tq_argmax_rows    index of each logit row's maximum (greedy sampling)
+ *   tq_linear         linear layer over many rows (fp32 on the bf16 matrix cores)
  *   tq_add_layernorm  residual add fused with the LayerNorm that follows it
  *   tq_skinny_linear  linear layer of at most 64 rows, LayerNorm / bias / GELU /
  *                     residual add fused in (small-batch decode steps)
@@ -334,6 +335,25 @@ size_t tq_paged_mixed_workspace_size(int32_t num_decode_seqs, int32_t num_heads,
  */
 tq_status tq_argmax_rows(int64_t* out, const float* logits, int64_t num_rows, int64_t num_cols,
                          int64_t row_stride, void* stream);
+
+/*
+ * A linear layer over many rows:
+ *
+ *   y[m] = epilogue( x[m] W^T + bias ),   0 <= m < M
+ *
+ * x is M rows of K floats (row stride x_stride elements), W is [N, K] contiguous, bias (may be
+ * null) has N entries, y is M rows of N floats (row stride y_stride). epilogue: 0 = none, 1 =
+ * tanh-form GELU. fp32 in, fp32 out, at fp32's precision (each operand split into three bf16
+ * numbers that add up to it, the products accumulated in fp32); infinities and NaN give what
+ * fp32 arithmetic gives. K a multiple of 32, at most 2^21; x and W 16-byte aligned, x_stride a
+ * multiple of 4 (y and bias: any alignment). Outputs must not alias inputs.
+ *
+ * Replaces nn.Linear over the packed rows of a prefill step (tokquay/model.py:62-63, :103-107)
+ * and the tied LM head of a large batch (:180-181).
+ */
+tq_status tq_linear(float* y, int64_t y_stride, const float* x, int64_t x_stride, int32_t M,
+                    const float* w, const float* bias, int32_t N, int32_t K,
+                    int32_t epilogue, void* stream);
 
 /*
  * Residual add + LayerNorm over rows of `cols` fp32 values:

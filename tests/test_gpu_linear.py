@@ -1,0 +1,116 @@
+"""tq_linear (linear layers over many rows) against float64, and the rule that sends calls to it.
+
+Tolerance: the kernel adds, per 16 of K, six exact bf16 products' sums into an fp32 accumulator (each
+addition off by at most 2^-24 of the running sum of |x w|) and drops products below 2^-24 |x w|, so an
+output is within (6 K / 16 + 4) 2^-24 sum |x w| of the exact value, plus the bias addition's rounding.
+GELU's slope is at most 1.13, its own evaluation good to a few 2^-24."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from tokquay_amd import ops
+
+EPS = 2.0**-24
+
+
+def _check(got, x, w, b, gelu=False):
+    x, w, got = x.double().cpu(), w.double().cpu(), got.double().cpu()
+    ref = x @ w.t()
+    bound = (6 * x.size(1) / 16 + 4) * EPS * (x.abs() @ w.abs().t())
+    if b is not None:
+        ref = ref + b.double().cpu()
+        bound = bound + EPS * ref.abs()
+    if gelu:
+        bound = 1.13 * bound + 16 * EPS * (1 + ref.abs())
+        ref = torch.nn.functional.gelu(ref, approximate="tanh")
+    assert ((got - ref).abs() <= bound + 1e-30).all(), float(((got - ref).abs() - bound).max())
+
+
+def _inputs(m, n, k, bias=True, seed=0):
+    g = torch.Generator().manual_seed(1000 * m + n + k + seed)
+    x, w = torch.randn(m, k, generator=g).cuda(), (torch.randn(n, k, generator=g) * 0.02).cuda()
+    return x, w, (torch.randn(n, generator=g) * 0.02).cuda() if bias else None
+
+
+# Rows around the 32-row waves and the 128- and 256-row tiles, columns around the 32-column blocks and
+# not a multiple of four, K of one, two, three and many steps; every tile shape is among them.
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 32), (1, 33, 64), (31, 64, 96), (33, 50, 768), (127, 96, 32), (129, 127, 64), (255, 2304, 768),
+    (257, 770, 96), (640, 2304, 768), (1000, 2304, 768), (1100, 3072, 64), (1987, 2304, 768), (2048, 3072, 96),
+    (2100, 768, 3072), (4097, 1024, 32), (66, 50257, 768),
+])  # fmt: skip
+@pytest.mark.parametrize("gelu", [False, True])
+def test_linear_matches_float64(m, n, k, gelu):
+    x, w, b = _inputs(m, n, k, bias=(m + n) % 3 != 0)
+    _check(ops._rows_linear(x, w, b, gelu), x, w, b, gelu)
+
+
+@pytest.mark.gpu
+def test_strided_rows_and_unaligned_outputs():
+    x, w, b = _inputs(300, 129, 96)
+    wide = torch.full((300, 132), 7.0, device="cuda")
+    wide[:, 4:100] = x
+    out = torch.full((300, 135), 5.0, device="cuda")
+    torch.ops.tokquay_amd.linear(out[:, 3:132], wide[:, 4:100], w, b, False)
+    _check(out[:, 3:132], x, w, b)
+    assert (out[:, :3] == 5).all() and (out[:, 132:] == 5).all()
+
+
+@pytest.mark.gpu
+def test_wide_ranges_stay_fp32():
+    """Rows and weights from 1e-30 to 1e30 keep fp32's precision (the limbs have fp32's exponents)."""
+    x, w, _ = _inputs(160, 96, 256, bias=False)
+    x = x * torch.logspace(-30, 15, 160).cuda()[:, None]
+    w = w * torch.logspace(-5, 18, 96).cuda()[:, None]
+    _check(ops._rows_linear(x, w, None, False), x, w, None)
+    eye = torch.eye(256, device="cuda")
+    y = ops._rows_linear(x, eye, None, False)
+    big = x.abs() > 1e-25  # the limbs of smaller values fall below the smallest normal number
+    assert torch.equal(y[big], x[big])
+
+
+@pytest.mark.gpu
+def test_non_finite_inputs_follow_fp32():
+    x, w, b = _inputs(200, 160, 128)
+    x[3, 5], x[40, 7], x[77, 0], x[150, 9] = float("inf"), float("-inf"), float("nan"), 3.4e38
+    w[11, 5], w[12, 9] = 0.0, 1e10
+    got = ops._rows_linear(x, w, b, False)
+    ref = torch.addmm(b.double(), x.double(), w.double().t()).float()
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
+    fin = ref.isfinite()
+    assert torch.equal(got[~fin & ~ref.isnan()], ref[~fin & ~ref.isnan()])
+    torch.testing.assert_close(got[fin], ref[fin], rtol=1e-4, atol=1e-4)
+
+
+def test_rule():
+    """Few tiles, K not in whole steps: the library; many: tq_linear."""
+    assert not ops.uses_rows_kernel(256, 2304, 768) and not ops.uses_rows_kernel(0, 2304, 768)
+    assert ops.uses_rows_kernel(640, 2304, 768) and ops.uses_rows_kernel(2048, 768, 3072)
+    assert ops.uses_rows_kernel(65, 50257, 768)
+    assert not ops.uses_rows_kernel(8192, 3072, 776) and not ops.uses_rows_kernel(8192, 3072, 0)
+
+
+@pytest.mark.gpu
+def test_calls_the_kernel_does_not_take_run_as_before(monkeypatch):
+    """Gradients, transforms, other types and layouts go the library's way, with its results."""
+    lin = torch.nn.Linear(64, 2304).cuda()
+    x = torch.randn(1024, 64, device="cuda")
+    taken = []
+    monkeypatch.setattr(ops, "_rows_linear", lambda *a: taken.append(a) or torch.empty(0))
+    y = ops.linear(x, lin)
+    assert y.requires_grad and not taken  # grad mode with trainable weights
+    with torch.no_grad():
+        ref = torch.nn.functional.linear(x, lin.weight, lin.bias)
+        for t in (x.t().contiguous().t(), torch.randn(1024, 66, device="cuda")[:, 1:65]):
+            out = ops.linear(t, lin)
+            torch.testing.assert_close(out, torch.nn.functional.linear(t, lin.weight, lin.bias), rtol=1e-4, atol=1e-4)
+        torch.testing.assert_close(torch.vmap(lambda r: ops.linear(r, lin))(x.expand(2, -1, -1))[1], ref, rtol=1e-4,
+                                   atol=1e-4)  # fmt: skip
+        half = torch.nn.Linear(64, 2304).cuda().half()
+        assert ops.linear(x.half(), half).dtype == torch.half
+        assert not taken
+        ops.linear(x, lin)
+        assert len(taken) == 1

@@ -139,6 +139,14 @@ SIGNATURES: dict[str, tuple] = {
             c_f32p, c_f32p, ctypes.c_int64, ctypes.c_int32, ctypes.c_float, ctypes.c_void_p,  # gamma, beta, rows, cols, eps, stream
         ],
     ),
+    "tq_linear": (
+        ctypes.c_int,
+        [
+            c_f32p, ctypes.c_int64, c_f32p, ctypes.c_int64, ctypes.c_int32,  # y, y_stride, x, x_stride, M
+            c_f32p, c_f32p, ctypes.c_int32, ctypes.c_int32,  # w, bias, N, K
+            ctypes.c_int32, ctypes.c_void_p,  # epilogue, stream
+        ],
+    ),
     "tq_skinny_linear": (
         ctypes.c_int,
         [

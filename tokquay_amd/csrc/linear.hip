@@ -1,0 +1,378 @@
+// Linear layers over many rows (prefill steps, mixed steps, the LM head of large batches):
+//
+//   y = epilogue( x W^T + b )      x [M, K], W [N, K] (nn.Linear layout), fp32 in, fp32 out
+//
+// as fp32 products on the bf16 matrix cores. Every fp32 operand is the exact sum of three
+// bf16 numbers (8 + 8 + 8 significant bits: each the rounded rest of the ones before), and
+//
+//   x w = x0 w0 + (x0 w1 + x1 w0) + (x0 w2 + x1 w1 + x2 w0) + terms below 2^-24 |x w|
+//
+// so six bf16 products, accumulated in fp32 by the MFMA, give the product to fp32's own
+// precision; the sum is the more exact for taking 16 k per accumulation instead of 4: against
+// float64, weights N(0, 0.02), rows N(0, 1): 2.1e-7 (K = 768) and 4.3e-7 (K = 3072) relative
+// where the fp32 MFMA GEMM of the library has 5.0e-7 and 9.9e-7. The fp32 MFMA peaks at 157
+// TFLOP/s on this GPU; bf16 runs ~1,200 (what a large library product reaches here, power
+// bound), a sixth of which is 200. The split costs no extra traffic: operands are read as
+// fp32 and split on the way in, nothing is kept between calls.
+//
+// Infinities, NaN and overflow: the split of a non-finite number (or of one that rounds past
+// the largest bf16) is NaN, so every output it touches comes out non-finite. A wave that sees
+// a non-finite accumulator computes its outputs again with plain fp32 FMAs, which gives them
+// IEEE's value.
+//
+// Work split: a workgroup of WM waves covers 32 WM rows x 32 NB columns; wave w owns rows
+// 32 w .. 32 w + 31 and all the columns, as NB accumulators of v_mfma_f32_32x32x16_bf16 (A = W,
+// B = X^T: lane (i, g) = (lane % 32, lane / 32) supplies row i, k octet g of a 16-wide k half).
+// Each wave reads and splits its own X rows straight into registers; W is read, split and
+// written to LDS once per workgroup, double buffered, one barrier per 32 of K.
+//  * 32x32x16 rather than 16x16x32: the split's VALU work (about four instructions per MFMA)
+//    hides behind it, while beside 16x16x32 it adds to the MFMA time (two waves a SIMD, 4 subs
+//    and 2 conversions per 32 cycles of MFMA: 35 cycles against 47).
+//  * X in registers: LDS is the next bound (reads 128 B, writes 64 B a clock and CU; three
+//    limbs are 6 B an element). With X in LDS too a 128 x 128 tile took 1.06 us per 32 of K,
+//    0.63 us of it LDS; this way 1.00 us. A wave's X loads have one row per lane, which the
+//    address unit takes at 16 B a clock; W's, four lanes a row, at 54, and W staged one row
+//    per lane cost 5-6 us of a 29 us tile.
+//  * W's fragments sit in LDS in the order the MFMA reads them, rows swizzled by the k octet,
+//    so neither side has bank conflicts.
+//  * A step's loads are issued two steps before they are split (one where the registers allow no
+//    more): weights come from HBM in a model's step, and one step is shorter than their latency.
+// Measured (GPU time, MI355X, weights evicted between calls) against the library's fp32 GEMM: 1,987
+// rows, [N, K] = [2304, 768] / [3072, 768] / [768, 3072] / [768, 768]: 76 / 78 / 86 / 27 -> 45 / 51 /
+// 67 / 20 us; 8,192 rows (operands resident): 221 / 280 / 266 / 85 -> 154 / 191 / 181 / 54 us (188-213
+// TFLOP/s of fp32 products, 1,130-1,280 of bf16 ones: power bound).
+//
+// Reference semantics: nn.Linear (tokquay/model.py:62-63, :103-104), the tanh GELU (:107), the
+// tied LM head (:180-181).
+
+#include <type_traits>
+
+#include "tq_internal.h"
+
+namespace tq {
+namespace {
+
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t uint32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kStep = 32;              // k per pipeline step
+constexpr int kXcds = 8;               // workgroup i is dispatched to XCD i % 8
+constexpr int kBufferWord3 = 0x00020000;  // raw buffer descriptor: 32-bit format, no swizzle
+
+enum Epilogue { kEpiBias = 0, kEpiGelu = 1 };
+
+struct LinearArgs {
+  float* y;
+  int64_t y_stride;
+  const float* x;
+  int64_t x_stride;
+  const float* w;
+  const float* bias;  // may be null
+  int32_t M, N, K;
+  int32_t m_tiles, n_tiles;
+  int32_t epilogue;
+  int32_t vec;  // rows of y and bias can be accessed four floats at a time
+};
+
+// v (tanh-form GELU): v / (1 + exp(-2u)) = 0.5 v (1 + tanh u), u = sqrt(2/pi) (v + 0.044715 v^3),
+// without the cancellation of 1 + tanh u for negative u.
+__device__ __forceinline__ float gelu(float v) {
+  const float u2 = -2.f * 0.7978845608028654f * (v + 0.044715f * v * v * v);
+  return v / (1.f + expf(u2));
+}
+
+// Eight fp32 values as three bf16 limbs: limb l holds the values' l-th bf16 (round to nearest of
+// what the limbs before left, an exact subtraction).
+__device__ __forceinline__ void split8(const floatx4& lo, const floatx4& hi, uint32x4 (&limb)[3]) {
+  float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+  for (int l = 0; l < 3; ++l) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const floatx2 pair = {v[2 * p], v[2 * p + 1]};
+      const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, bf16x2));
+      limb[l][p] = u;
+      if (l < 2) {
+        v[2 * p] -= __uint_as_float(u << 16);
+        v[2 * p + 1] -= __uint_as_float(u & 0xffff0000u);
+      }
+    }
+  }
+}
+
+__device__ __forceinline__ void load8(const __amdgpu_buffer_rsrc_t& d, floatx4 (&r)[2], uint32_t offset, int32_t k) {
+  r[0] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(d, offset, k * 4, 0));
+  r[1] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(d, offset + 16, k * 4, 0));
+}
+
+template <int WM, int NB, int DEPTH>
+__global__ __launch_bounds__(kWave* WM, WM == 8 ? 1 : 2) void linear_kernel(const LinearArgs a) {
+  constexpr int BM = 32 * WM, BN = 32 * NB;
+  constexpr int kUnits = 2 * NB;                     // staging units: 16 rows of W each
+  constexpr int kOwn = (kUnits + WM - 1) / WM;       // units a wave stages (the last ones may repeat)
+  constexpr int kPad = 36;                           // row stride of the output transpose, conflict free
+  struct Stage {
+    uint32x4 w[2][NB][2][3][kWave];  // [buffer][column block][k half][limb][lane]
+  };
+  struct Out {
+    float rows[WM][32][kPad];  // a 32 x 32 block of each wave
+  };
+  __shared__ union {
+    Stage st;
+    Out out;
+  } s;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int i = lane & 31, g = lane >> 5;
+
+  // Each XCD takes a contiguous run of tiles along the shorter of M and N, so that of the two
+  // operands it reads the smaller one whole and about an eighth of the other.
+  const int total = a.m_tiles * a.n_tiles;
+  const int q = total / kXcds, rem = total % kXcds, xcd = blockIdx.x % kXcds;
+  const int p = xcd * q + min(xcd, rem) + blockIdx.x / kXcds;
+  const bool rows_first = a.M < a.N;
+  const int minor = rows_first ? a.m_tiles : a.n_tiles;
+  const int hi = p / minor, lo = p - hi * minor;
+  const int m_tile = rows_first ? lo : hi, n_tile = rows_first ? hi : lo;
+  const int m0 = m_tile * BM + 32 * wave, n0 = n_tile * BN;
+
+  // Descriptors on the wave's rows of X and the tile's rows of W: loads past the last row give 0.
+  const int x_rows = max(0, min(32, a.M - m0)), w_rows = min(BN, a.N - n0);
+  const __amdgpu_buffer_rsrc_t xd = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(a.x + (int64_t)min(m0, a.M - 1) * a.x_stride), (short)0,
+      x_rows > 0 ? (int32_t)(((x_rows - 1) * a.x_stride + a.K) * 4) : 0, kBufferWord3);
+  const __amdgpu_buffer_rsrc_t wd = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.w + (int64_t)n0 * a.K),
+                                                                      (short)0, w_rows * a.K * 4, kBufferWord3);
+  const uint32_t x_off = (uint32_t)(i * a.x_stride + 8 * g) * 4u;  // row i, octet g of each k half
+  // Staging: unit rows lane / 4, k octet lane % 4 (k half octet / 2).
+  const int sr = lane >> 2, so = lane & 3;
+  uint32_t w_off[kOwn];
+  int w_unit[kOwn];
+#pragma unroll
+  for (int u = 0; u < kOwn; ++u) {
+    w_unit[u] = min(wave + WM * u, kUnits - 1);  // a repeated unit stores the same values again
+    w_off[u] = (uint32_t)((16 * w_unit[u] + sr) * a.K + 8 * so) * 4u;
+  }
+  // Slot of (row, octet) in a fragment: 32 (octet % 2) + (row ^ 4 octet).
+  const int slot[2] = {32 * g + (i ^ (g << 2)), 32 * g + (i ^ ((2 + g) << 2))};
+
+  floatx16 acc[NB];
+#pragma unroll
+  for (int n = 0; n < NB; ++n)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[n][r] = 0.f;
+  // Operands as loaded, [step % DEPTH]: a step's loads are issued DEPTH steps before it is split.
+  floatx4 xr[DEPTH][2][2], wr[DEPTH][kOwn][2];
+  uint32x4 xl[2][2][3];           // [step parity][k half][limb]
+  auto stage = [&](int buf, const floatx4(&raw)[2], int u) {
+    uint32x4 l[3];
+    split8(raw[0], raw[1], l);
+    const int row = (16 * (w_unit[u] & 1) + sr) ^ (so << 2);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) s.st.w[buf][w_unit[u] >> 1][so >> 1][t][32 * (so & 1) + row] = l[t];
+  };
+
+  // The six products, smallest first: limb of W, limb of X.
+  constexpr int kW[6] = {2, 0, 1, 1, 0, 0}, kX[6] = {0, 2, 1, 0, 1, 0};
+  // One step: the MFMAs of step parity CUR; between them the next step's operands are split
+  // (W's into the other buffer) and the step after's loads (at k_next) are issued. LAST: nothing
+  // to prepare. The regions (column block, k half) are fenced from each other so that every
+  // region keeps its own share of the split work between its MFMAs.
+  auto step = [&](auto cur, auto last, int32_t k_next) {
+    constexpr int CUR = decltype(cur)::value;
+    constexpr bool LAST = decltype(last)::value;
+    constexpr int kSplits = kOwn + 2, kRegions = 2 * NB;
+    constexpr int kRaw = DEPTH == 2 ? CUR ^ 1 : 0;  // where the next step's operands are
+    bf16x8 w[2][3];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) w[0][t] = __builtin_bit_cast(bf16x8, s.st.w[CUR][0][0][t][slot[0]]);
+#pragma unroll
+    for (int r = 0; r < kRegions; ++r) {
+      if (r + 1 < kRegions) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+          w[(r + 1) & 1][t] = __builtin_bit_cast(bf16x8, s.st.w[CUR][(r + 1) / 2][(r + 1) & 1][t][slot[(r + 1) & 1]]);
+      }
+      if constexpr (!LAST) {
+#pragma unroll
+        for (int u = r * kSplits / kRegions; u < (r + 1) * kSplits / kRegions; ++u) {
+          if (u < kOwn) {
+            stage(CUR ^ 1, wr[kRaw][u], u);
+            load8(wd, wr[kRaw][u], w_off[u], k_next);
+          } else {
+            floatx4(&raw)[2] = xr[kRaw][u - kOwn];
+            split8(raw[0], raw[1], xl[CUR ^ 1][u - kOwn]);
+            load8(xd, raw, x_off + 64 * (u - kOwn), k_next);
+          }
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < 6; ++t)
+        acc[r / 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            w[r & 1][kW[t]], __builtin_bit_cast(bf16x8, xl[CUR][r & 1][kX[t]]), acc[r / 2], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (!LAST) __syncthreads();
+  };
+
+  const int steps = a.K / kStep;
+  const int32_t k_end = (steps - 1) * kStep;
+  auto load_step = [&](int at, int32_t k) {
+#pragma unroll
+    for (int u = 0; u < kOwn; ++u) load8(wd, wr[at][u], w_off[u], k);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) load8(xd, xr[at][h], x_off + 64 * h, k);
+  };
+  load_step(0, 0);
+  if constexpr (DEPTH == 2) load_step(1, min(kStep, k_end));
+#pragma unroll
+  for (int u = 0; u < kOwn; ++u) stage(0, wr[0][u], u);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) split8(xr[0][h][0], xr[0][h][1], xl[0][h]);
+  load_step(0, min(DEPTH * kStep, k_end));
+  __syncthreads();
+  using Even = std::integral_constant<int, 0>;
+  using Odd = std::integral_constant<int, 1>;
+  auto ahead = [&](int t) { return min((t + 1 + DEPTH) * kStep, k_end); };  // past the end: the last step again
+  int st = 0;
+  for (; st + 2 < steps; st += 2) {
+    step(Even{}, std::false_type{}, ahead(st));
+    step(Odd{}, std::false_type{}, ahead(st + 1));
+  }
+  if (st + 2 == steps) {
+    step(Even{}, std::false_type{}, k_end);
+    step(Odd{}, std::true_type{}, 0);
+  } else {
+    step(Even{}, std::true_type{}, 0);
+  }
+
+  auto finish = [&](float v) { return a.epilogue == kEpiGelu ? gelu(v) : v; };
+  float probe = 0.f;  // NaN once any accumulator is infinite or NaN
+#pragma unroll
+  for (int n = 0; n < NB; ++n)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) probe = fmaf(acc[n][r], 0.f, probe);
+  const bool plain = __builtin_amdgcn_ballot_w64(probe != probe) != 0;  // uniform: see the top of the file
+  __syncthreads();  // the stage buffers become the output blocks
+  if (plain) {
+    for (int e = lane; e < 32 * BN; e += kWave) {
+      const int m = m0 + e / BN, c = n0 + e % BN;
+      if (m >= a.M || c >= a.N) continue;
+      const float* xp = a.x + (int64_t)m * a.x_stride;
+      const float* wp = a.w + (int64_t)c * a.K;
+      float v = 0.f;
+      for (int k = 0; k < a.K; ++k) v = fmaf(xp[k], wp[k], v);
+      a.y[(int64_t)m * a.y_stride + c] = finish(a.bias != nullptr ? v + a.bias[c] : v);
+    }
+    return;
+  }
+  // Each 32 x 32 block goes through the wave's own LDS rows, so that the stores cover whole
+  // 128-byte runs of y (lane: row 8 t + lane / 8, columns 4 (lane % 8) ..).
+  const int oc = 4 * (lane & 7);
+#pragma unroll
+  for (int n = 0; n < NB; ++n) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      *reinterpret_cast<floatx4*>(&s.out.rows[wave][i][8 * r + 4 * g]) =
+          floatx4{acc[n][4 * r], acc[n][4 * r + 1], acc[n][4 * r + 2], acc[n][4 * r + 3]};
+    const int c = n0 + 32 * n + oc;
+    floatx4 b = {0.f, 0.f, 0.f, 0.f};
+    if (a.bias != nullptr) {
+      if (a.vec) {
+        if (c < a.N) b = *reinterpret_cast<const floatx4*>(a.bias + c);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) b[e] = c + e < a.N ? a.bias[c + e] : 0.f;
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int row = 8 * t + (lane >> 3);
+      floatx4 v = *reinterpret_cast<const floatx4*>(&s.out.rows[wave][row][oc]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = finish(v[e] + b[e]);
+      if (m0 + row >= a.M) continue;
+      float* yp = a.y + (int64_t)(m0 + row) * a.y_stride + c;
+      if (a.vec) {
+        if (c < a.N) *reinterpret_cast<floatx4*>(yp) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (c + e < a.N) yp[e] = v[e];
+      }
+    }
+  }
+}
+
+template <int WM, int NB, int DEPTH>
+void launch(LinearArgs a, hipStream_t s) {
+  a.m_tiles = (a.M + 32 * WM - 1) / (32 * WM);
+  a.n_tiles = (a.N + 32 * NB - 1) / (32 * NB);
+  hipLaunchKernelGGL((linear_kernel<WM, NB, DEPTH>), dim3((unsigned)(a.m_tiles * a.n_tiles)), dim3(kWave * WM), 0, s, a);
+}
+
+// Tile shapes and what one tile takes per 32 of K alone on a CU (ns, measured at K = 3072). A CU
+// gains nothing from a second resident tile (LDS and the matrix cores are busy already), so a
+// launch takes ceil(tiles / 256) of them in a row: the shape with the least rounds x time wins.
+// (E.g. 1,987 rows x 2,304: 128 x 64 tiles need three rounds, 52 us; 256 x 96 one, 43 us.)
+struct TileShape {
+  int wm, nb;
+  int step_ns;
+};
+constexpr TileShape kShapes[] = {{4, 1, 575}, {4, 2, 630}, {4, 3, 885}, {4, 4, 1000}, {8, 3, 1235}, {8, 4, 1630}};
+
+const TileShape& choose_shape(int64_t M, int64_t N) {
+  constexpr int64_t kCus = 256;
+  const TileShape* best = nullptr;
+  int64_t best_ns = 0;
+  for (const TileShape& t : kShapes) {
+    const int64_t tiles = ((M + 32 * t.wm - 1) / (32 * t.wm)) * ((N + 32 * t.nb - 1) / (32 * t.nb));
+    const int64_t ns = (tiles + kCus - 1) / kCus * t.step_ns;
+    if (best == nullptr || ns < best_ns) best = &t, best_ns = ns;
+  }
+  return *best;
+}
+
+}  // namespace
+}  // namespace tq
+
+extern "C" tq_status tq_linear(float* y, int64_t y_stride, const float* x, int64_t x_stride, int32_t M, const float* w,
+                               const float* bias, int32_t N, int32_t K, int32_t epilogue, void* stream) {
+  using namespace tq;
+  if (M < 0 || N < 1 || K < 1 || epilogue < 0 || epilogue > 1) return TQ_ERR_INVALID_ARGUMENT;
+  // 32-bit offsets inside a tile; K in whole steps.
+  if (K % kStep != 0 || (int64_t)K * 4 * 256 > 0x7fffffffLL || x_stride * 4 * 256 > 0x7fffffffLL)
+    return TQ_ERR_UNSUPPORTED;
+  if (M == 0) return TQ_OK;
+  if (y == nullptr || x == nullptr || w == nullptr) return TQ_ERR_INVALID_ARGUMENT;
+  if (x_stride < K || y_stride < N) return TQ_ERR_INVALID_ARGUMENT;
+  if (((uintptr_t)x | (uintptr_t)w) % 16 != 0 || x_stride % 4 != 0) return TQ_ERR_INVALID_ARGUMENT;
+  if (((int64_t)M + 127) / 128 * (((int64_t)N + 31) / 32) > 0x7fffffffLL) return TQ_ERR_UNSUPPORTED;
+  LinearArgs a = {};
+  a.y = y;
+  a.y_stride = y_stride;
+  a.x = x;
+  a.x_stride = x_stride;
+  a.w = w;
+  a.bias = bias;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.epilogue = epilogue;
+  a.vec = N % 4 == 0 && y_stride % 4 == 0 && ((uintptr_t)y | (uintptr_t)bias) % 16 == 0;
+  hipStream_t s = (hipStream_t)stream;
+  const TileShape& t = choose_shape(M, N);
+  switch (t.wm * 10 + t.nb) {
+    case 41: launch<4, 1, 2>(a, s); break;
+    case 42: launch<4, 2, 2>(a, s); break;
+    case 43: launch<4, 3, 2>(a, s); break;
+    case 44: launch<4, 4, 1>(a, s); break;
+    case 83: launch<8, 3, 2>(a, s); break;
+    default: launch<8, 4, 2>(a, s); break;
+  }
+  return check_launch();
+}

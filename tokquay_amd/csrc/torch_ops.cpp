@@ -281,6 +281,31 @@ void argmax_rows(const at::Tensor& logits, at::Tensor out) {
         "tq_argmax_rows");
 }
 
+void linear(at::Tensor out, const at::Tensor& x, const at::Tensor& weight, const c10::optional<at::Tensor>& bias,
+            bool gelu) {
+  const char* op = "tokquay_amd::linear";
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kFloat && x.dim() == 2 && (x.size(1) <= 1 || x.stride(1) == 1), op,
+              ": x must be a float32 [rows, K] tensor on a HIP device with contiguous rows");
+  const int64_t M = x.size(0), K = x.size(1);
+  TORCH_CHECK(M <= 1 || x.stride(0) >= K, op, ": x's rows overlap");
+  TORCH_CHECK(weight.device() == x.device() && weight.scalar_type() == at::kFloat && weight.dim() == 2 &&
+                  weight.size(1) == K && weight.is_contiguous(),
+              op, ": weight must be a contiguous float32 [N, K] tensor on x's device");
+  const int64_t N = weight.size(0);
+  TORCH_CHECK(!bias.has_value() || (bias->device() == x.device() && bias->scalar_type() == at::kFloat &&
+                                    bias->dim() == 1 && bias->size(0) == N && bias->is_contiguous()),
+              op, ": bias must be a contiguous float32 [N] tensor on x's device");
+  TORCH_CHECK(out.device() == x.device() && out.scalar_type() == at::kFloat && out.dim() == 2 && out.size(0) == M &&
+                  out.size(1) == N && (N <= 1 || out.stride(1) == 1),
+              op, ": out must be a float32 [rows, N] tensor on x's device with contiguous rows");
+  TORCH_CHECK(M <= 1 || out.stride(0) >= N, op, ": out's rows overlap");
+  TORCH_CHECK(M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX, op, ": sizes past int32");
+  check(tq_linear(out.data_ptr<float>(), M > 1 ? out.stride(0) : N, x.data_ptr<float>(), M > 1 ? x.stride(0) : K,
+                  (int32_t)M, weight.data_ptr<float>(), ptr<float>(bias), (int32_t)N, (int32_t)K, gelu ? 1 : 0,
+                  stream_of(x)),
+        "tq_linear");
+}
+
 }  // namespace
 
 TORCH_LIBRARY(tokquay_amd, m) {
@@ -300,6 +325,7 @@ TORCH_LIBRARY(tokquay_amd, m) {
   m.def("paged_gather(Tensor(a!) k_out, Tensor(b!) v_out, Tensor pool, int layer, Tensor block_tables, "
         "Tensor(c!)? d_error) -> ()");
   m.def("argmax_rows(Tensor logits, Tensor(a!) out) -> ()");
+  m.def("linear(Tensor(a!) out, Tensor x, Tensor weight, Tensor? bias, bool gelu) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(tokquay_amd, CUDA, m) {
@@ -310,4 +336,5 @@ TORCH_LIBRARY_IMPL(tokquay_amd, CUDA, m) {
   m.impl("paged_mixed", &paged_mixed);
   m.impl("paged_gather", &paged_gather);
   m.impl("argmax_rows", &argmax_rows);
+  m.impl("linear", &linear);
 }

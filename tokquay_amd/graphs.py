@@ -168,7 +168,7 @@ class DecodeGraphs:
             # residual add fused in.
             logits = m.skinny_logits(x, view)
         else:
-            logits = m.trunk(None, None, view, embedded=x) @ m.wte.weight.T
+            logits = ops.lm_head(m.trunk(None, None, view, embedded=x), m.wte.weight)
         ops.argmax_rows(logits, out=s.tokens[:rows])
         return logits
 

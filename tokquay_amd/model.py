@@ -139,7 +139,7 @@ class GPT2(nn.Module):
         if x.shape[0] <= ops.SKINNY_LM_HEAD_MAX_ROWS:
             return ops.skinny_linear(x, self.wte.weight, None, ln=(self.ln_f.weight, self.ln_f.bias, self.ln_f.eps))
         _, h = ops.add_layernorm(x, None, self.ln_f.weight, self.ln_f.bias, self.ln_f.eps, x_out=x)
-        return h @ self.wte.weight.T
+        return ops.lm_head(h, self.wte.weight)
 
     def skinny_greedy(self, x: torch.Tensor, cache, out: torch.Tensor) -> torch.Tensor:
         """Greedy ids ``[M]`` of ``M <= ops.SKINNY_LM_HEAD_MAX_ROWS`` rows into ``out`` without logits:
@@ -163,8 +163,8 @@ class GPT2(nn.Module):
         ids = input_ids.reshape(-1).index_select(0, cache.token_index)  # [N] real tokens only
         h = self.trunk(ids, cache.packed_positions, cache)  # positions of real tokens are < n_positions
         if last_only:
-            return (h.index_select(0, cache.last_rows) @ self.wte.weight.T)[:, None]  # tied LM head, [B, 1, V]
-        logits = h @ self.wte.weight.T  # [N, vocab]
+            return ops.lm_head(h.index_select(0, cache.last_rows), self.wte.weight)[:, None]  # tied LM head, [B, 1, V]
+        logits = ops.lm_head(h, self.wte.weight)  # [N, vocab]
         full = logits.new_zeros(B * T, logits.size(-1))
         full[cache.token_index] = logits
         return full.view(B, T, -1)

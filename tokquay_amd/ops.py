@@ -531,13 +531,66 @@ def uses_nn_layout(rows: int, out_features: int, in_features: int, gelu: bool) -
     return (rows, out_features, in_features, gelu) in GEMM_NN_SHAPES
 
 
+# tq_linear from this many 128 x 64 output tiles on: below, too few of the 256 CUs get a tile and the
+# library's small tiles and K splits win. Measured us (library -> tq_linear, [rows, N, K]): [320, 3072, 768]
+# 144 tiles 15.8 -> 18.6; [768, 1600, 1600] 150 tiles 33.8 -> 34.5; [1280, 1024, 1024] 160 tiles 24.9 -> 24.1;
+# [640, 2304, 768] 180 tiles 25.6 -> 19.2; [2048, 768, 768] 192 tiles 26.1 -> 19.9; [2048, 768, 3072] 192 tiles
+# 78.8 -> 66.4; [65, 50257, 768] 786 tiles 69.8 -> 52.7; [8192, 3072, 768] 3,072 tiles 280 -> 191.
+ROWS_KERNEL_MIN_TILES = 160
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
+def uses_rows_kernel(rows: int, out_features: int, in_features: int) -> bool:
+    """Whether a linear layer of these sizes runs on ``tq_linear`` (else on the library GEMM)."""
+    return (((rows + 127) >> 7) * ((out_features + 63) >> 6) >= ROWS_KERNEL_MIN_TILES
+            and in_features % 32 == 0 and in_features > 0)  # fmt: skip
+
+
+def _rows_kernel_takes(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None) -> bool:
+    """Whether ``x @ w.T + bias`` may go to ``tq_linear``: enough tiles (``uses_rows_kernel``), plain
+    float32 tensors on one HIP device in the layout it reads, and nothing that must see torch's own
+    product (a gradient, a functorch transform, forward-mode AD, a tensor subclass)."""
+    n, k = w.shape
+    if not uses_rows_kernel(x.size(0), n, k):  # most small calls end here: the cheapest test first
+        return False
+    if x.dim() != 2 or x.size(1) != k:
+        return False
+    ts = (x, w) if bias is None else (x, w, bias)
+    if any(type(t) not in _TENSORS or t.dtype != torch.float32 or t.device != x.device for t in ts):
+        return False
+    if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
+        return False
+    if torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    return (w.is_contiguous() and x.stride(1) == 1 and x.stride(0) >= k and x.stride(0) % 4 == 0
+            and x.stride(0) < 1 << 21 and k <= 1 << 21
+            and (bias is None or (bias.dim() == 1 and bias.size(0) == n and bias.is_contiguous()))
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)  # fmt: skip
+
+
+def _rows_linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, gelu: bool) -> torch.Tensor:
+    out = torch.empty(x.size(0), w.size(0), dtype=torch.float32, device=x.device)
+    _op("linear", out, x, w, bias, gelu)
+    return out
+
+
+def lm_head(h: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """Logits ``h @ weight.T`` of the tied LM head (tokquay/model.py:180-181): ``tq_linear`` over many
+    rows, else the library GEMM."""
+    if h.is_cuda and _rows_kernel_takes(h, weight, None):
+        return _rows_linear(h, weight, None, False)
+    return h @ weight.T
+
+
 def linear(x: torch.Tensor, layer: torch.nn.Linear, gelu: bool = False) -> torch.Tensor:
-    """``x @ layer.weight.T + layer.bias`` (then the tanh GELU when ``gelu``) through hipBLASLt, in
-    the weight layout ``GEMM_NN_SHAPES`` names for this shape. On the CPU: torch's ``F.linear`` and
-    the tanh GELU."""
+    """``x @ layer.weight.T + layer.bias`` (then the tanh GELU when ``gelu``): ``tq_linear`` over many
+    rows (``uses_rows_kernel``), else hipBLASLt in the weight layout ``GEMM_NN_SHAPES`` names for
+    this shape. On the CPU: torch's ``F.linear`` and the tanh GELU."""
     if not x.is_cuda:
         y = torch.nn.functional.linear(x, layer.weight, layer.bias)
         return torch.nn.functional.gelu(y, approximate="tanh") if gelu else y
+    if _rows_kernel_takes(x, layer.weight, layer.bias):
+        return _rows_linear(x, layer.weight, layer.bias, gelu)
     out_f, in_f = layer.weight.shape
     nn_layout = uses_nn_layout(x.shape[0], out_f, in_f, gelu)
     w = transposed_weight(layer) if nn_layout else layer.weight.t()

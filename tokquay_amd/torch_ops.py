@@ -1,6 +1,6 @@
 """``torch.ops.tokquay_amd.*``: the paged-attention entry points as torch operators.
 
-``csrc/torch_ops.cpp`` (built into ``_torch_ops.so`` next to ``libtokquay_amd.so``) registers seven
+``csrc/torch_ops.cpp`` (built into ``_torch_ops.so`` next to ``libtokquay_amd.so``) registers eight
 out-variant operators with torch's dispatcher; each is a thin call into the C ABI on the current
 HIP stream. This module loads that library and registers the operators' fake (shape-only)
 implementations, so programs that record torch calls (``make_fx``, FX graphs on fake tensors)
@@ -20,6 +20,7 @@ or entries, overlapping rows:
 * ``paged_gather(k_out!, v_out!, pool, layer, block_tables, d_error!?)`` (the reference view's
   gathered copy)
 * ``argmax_rows(logits, out!)``
+* ``linear(out!, x, weight, bias?, gelu)``
 
 (``!``: written in place.) ``tokquay_amd.ops`` checks the tensors with the reference's messages
 and calls these operators; there is no fallback when the library is missing.
@@ -34,7 +35,7 @@ import torch
 from tokquay_amd.build import TORCH_OPS_PATH
 
 OPS = ("cache_write", "paged_decode", "paged_decode_write", "paged_prefill", "paged_mixed", "paged_gather",
-       "argmax_rows")
+       "argmax_rows", "linear")
 
 _loaded = False
 
@@ -210,6 +211,30 @@ def _fake_argmax_rows(logits, out):
     if not (out.device == logits.device and out.dtype == torch.int64 and out.is_contiguous()
             and out.numel() >= logits.size(0)):  # fmt: skip
         _fail(op, "out must be a contiguous int64 tensor with one entry per row, on the logits' device")
+
+
+def _fake_linear(out, x, weight, bias, gelu):
+    op = "linear"
+
+    def matrix(t, cols=None):
+        return (t.dtype == torch.float32 and t.dim() == 2 and (cols is None or t.size(1) == cols)
+                and (t.size(1) <= 1 or t.stride(1) == 1))  # fmt: skip
+
+    if not (x.is_cuda and matrix(x)):
+        _fail(op, "x must be a float32 [rows, K] tensor on a HIP device with contiguous rows")
+    rows, k = x.shape
+    if rows > 1 and x.stride(0) < k:
+        _fail(op, "x's rows overlap")
+    if not (weight.device == x.device and matrix(weight, k) and weight.is_contiguous()):
+        _fail(op, "weight must be a contiguous float32 [N, K] tensor on x's device")
+    n = weight.size(0)
+    if bias is not None and not (bias.device == x.device and bias.dtype == torch.float32 and bias.shape == (n,)
+                                 and bias.is_contiguous()):  # fmt: skip
+        _fail(op, "bias must be a contiguous float32 [N] tensor on x's device")
+    if not (out.device == x.device and matrix(out, n) and out.size(0) == rows):
+        _fail(op, "out must be a float32 [rows, N] tensor on x's device with contiguous rows")
+    if rows > 1 and out.stride(0) < n:
+        _fail(op, "out's rows overlap")
 
 
 FAKES = {name: globals()[f"_fake_{name}"] for name in OPS}
