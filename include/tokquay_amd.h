@@ -286,7 +286,8 @@ tq_status tq_paged_prefill(float* out, int64_t out_row_stride,
  * sequences must not share a pool slot that the decode rows write.
  *
  * The decode rows' waves and the prefill tiles run side by side in one grid, so HBM
- * streaming and MFMA work overlap and the launch cost is paid once. Every output row is
+ * streaming and MFMA work overlap and the launch cost is paid once (with thousands of
+ * prefill rows the call makes the two launches itself: they are faster then). Every output row is
  * bit-identical to the corresponding single-kind call's (for the decode rows: the one with
  * the same partition length; partition_tokens = 0 lets this call choose its own, so compare
  * with an explicit one). With no prefill rows this is tq_paged_decode_write, with no decode

@@ -1,0 +1,105 @@
+"""Prefill launches with many query rows (128-query workgroups on the bf16 matrix cores) against the
+oracle's gather path and float64 brute force, at the edges of their tiles: query counts around 32 and
+128, key counts around 32 and past one refresh of 64 block ids, starts inside blocks, block sizes 16
+and 32. 64 heads give a launch the rows it needs from short sequences."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from tests.paged_cases import ATOL, RTOL, Scenario
+from tokquay_amd import ops
+from tokquay_amd.kv_cache import PagedBatch
+
+H = 64
+SHAPES = [
+    ([0, 0, 0, 0, 0], [256, 200, 129, 128, 97]),
+    ([1000, 37, 300, 5], [300, 257, 31, 255]),
+    ([0, 64, 511, 15, 16], [385, 161, 160, 159, 2]),
+    ([3, 200, 31, 2000], [128, 127, 140, 250]),
+]
+
+
+def _run_alone(sc, b):
+    """Sequence b's attention as a launch of its own (few rows: the 16-row kernels)."""
+    one = PagedBatch(sc.gpu_pool, sc.block_size, [sc.tables[b]], [sc.starts[b]], [sc.new_lens[b]])
+    rows = sc.rows[b]
+    out = torch.empty(len(rows), sc.C, device="cuda")
+    ops.paged_prefill(out, sc.qkv[rows, : sc.C], sc.gpu_pool, 0, one.prefill_block_tables, one.prefill_cu_seqlens,
+                      one.prefill_start, one.prefill_max_q)  # fmt: skip
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("starts,lens", SHAPES)
+@pytest.mark.parametrize("bs", [16, 32])
+def test_matches_the_oracle(starts, lens, bs):
+    sc = Scenario(starts, lens, block_size=bs, n_head=H, seed=sum(lens))
+    pool_ref, out_ref = sc.reference()
+    pool, out, batch = sc.run_product()
+    assert torch.equal(pool, pool_ref)
+    torch.testing.assert_close(out, sc.packed_reference(out_ref, batch.token_index), rtol=RTOL, atol=ATOL)
+    at = 0
+    for want in sc.brute_force(pool_ref):
+        got = out[at : at + want.shape[0]].view(-1, H, 64)
+        torch.testing.assert_close(got.double(), torch.from_numpy(want), rtol=RTOL, atol=ATOL)
+        at += want.shape[0]
+    # The launch is the wide one: its bits are not those of the sequences launched alone.
+    sc.gpu_pool, sc.qkv = pool.cuda(), sc.packed_qkv(batch.token_index).cuda()
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    sc.rows = [torch.arange(cu[b], cu[b + 1], device="cuda") for b in range(len(lens))]
+    alone = torch.cat([_run_alone(sc, b) for b in range(len(lens))]).cpu()
+    torch.testing.assert_close(out, alone, rtol=RTOL, atol=ATOL)
+    assert not torch.equal(out, alone)
+
+
+@pytest.mark.gpu
+def test_dispatch_order_keeps_the_bits_and_bad_metadata_is_reported():
+    sc = Scenario(*SHAPES[0], n_head=H)
+    pool, out, batch = sc.run_product()
+    qkv, gpu_pool = sc.packed_qkv(batch.token_index).cuda(), pool.cuda()
+    err = torch.zeros(1, dtype=torch.int32, device="cuda")
+
+    def run(tables, order):
+        got = torch.empty(qkv.size(0), sc.C, device="cuda")
+        ops.paged_prefill(got, qkv[:, : sc.C], gpu_pool, 0, tables, batch.prefill_cu_seqlens, batch.prefill_start,
+                          batch.prefill_max_q, d_error=err, seq_order=order)  # fmt: skip
+        return got.cpu()
+
+    for perm in ([4, 3, 2, 1, 0], [2, 0, 4, 1, 3]):
+        assert torch.equal(run(batch.prefill_block_tables, torch.tensor(perm, dtype=torch.int32, device="cuda")), out)
+    assert torch.equal(run(batch.prefill_block_tables, None), out) and int(err) == 0
+    tables = batch.prefill_block_tables.clone()
+    tables[1, 3] = gpu_pool.size(0)  # a block past the pool: its keys count as zeros, the others run on
+    got = run(tables, None)
+    assert int(err) == 1 and got.isfinite().all()
+    keep = torch.ones(out.size(0), dtype=torch.bool)
+    keep[256 + 48 : 456] = False  # sequence 1's rows from the bad block's first position on
+    assert torch.equal(got[keep], out[keep])
+
+
+@pytest.mark.gpu
+def test_non_finite_keys_follow_fp32_softmax():
+    """An infinite key gives a query that sees it what fp32 softmax gives (NaN, or no weight), and does
+    not reach the queries before it."""
+    starts, lens = SHAPES[0]
+    sc = Scenario(starts, lens, n_head=H)
+    sc.k[0, 3, 100, 7] = float("inf")
+    sc.k[2, 5, 40, 0] = float("-inf")
+    pool, out, batch = sc.run_product()
+    clean, want, _ = Scenario(starts, lens, n_head=H).run_product()
+    want = want.double().view(-1, H, 64).clone()
+    at = [0, 256, 456, 585, 713]
+    for b, h, pos in ((0, 3, 100), (2, 5, 40)):
+        q, k, v = (t[b, h].double() for t in (sc.q, sc.k, sc.v))
+        for t in range(pos, lens[b]):
+            p = torch.softmax(k[: t + 1] @ q[t] / math.sqrt(64), 0)
+            want[at[b] + t, h] = p @ v[: t + 1]
+    got = out.double().view(-1, H, 64)
+    assert want.isnan().any() and want[at[0] + 100 : at[0] + 256, 3].isfinite().any()
+    torch.testing.assert_close(got, want, rtol=RTOL, atol=ATOL, equal_nan=True)

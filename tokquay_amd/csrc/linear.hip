@@ -47,17 +47,11 @@
 
 #include <type_traits>
 
+#include "split_bf16.h"
 #include "tq_internal.h"
 
 namespace tq {
 namespace {
-
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t uint32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kStep = 32;              // k per pipeline step
 constexpr int kXcds = 8;               // workgroup i is dispatched to XCD i % 8
@@ -83,25 +77,6 @@ struct LinearArgs {
 __device__ __forceinline__ float gelu(float v) {
   const float u2 = -2.f * 0.7978845608028654f * (v + 0.044715f * v * v * v);
   return v / (1.f + expf(u2));
-}
-
-// Eight fp32 values as three bf16 limbs: limb l holds the values' l-th bf16 (round to nearest of
-// what the limbs before left, an exact subtraction).
-__device__ __forceinline__ void split8(const floatx4& lo, const floatx4& hi, uint32x4 (&limb)[3]) {
-  float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-#pragma unroll
-  for (int l = 0; l < 3; ++l) {
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const floatx2 pair = {v[2 * p], v[2 * p + 1]};
-      const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, bf16x2));
-      limb[l][p] = u;
-      if (l < 2) {
-        v[2 * p] -= __uint_as_float(u << 16);
-        v[2 * p + 1] -= __uint_as_float(u & 0xffff0000u);
-      }
-    }
-  }
 }
 
 __device__ __forceinline__ void load8(const __amdgpu_buffer_rsrc_t& d, floatx4 (&r)[2], uint32_t offset, int32_t k) {
@@ -176,8 +151,6 @@ __global__ __launch_bounds__(kWave* WM, WM == 8 ? 1 : 2) void linear_kernel(cons
     for (int t = 0; t < 3; ++t) s.st.w[buf][w_unit[u] >> 1][so >> 1][t][32 * (so & 1) + row] = l[t];
   };
 
-  // The six products, smallest first: limb of W, limb of X.
-  constexpr int kW[6] = {2, 0, 1, 1, 0, 0}, kX[6] = {0, 2, 1, 0, 1, 0};
   // One step: the MFMAs of step parity CUR; between them the next step's operands are split
   // (W's into the other buffer) and the step after's loads (at k_next) are issued. LAST: nothing
   // to prepare. The regions (column block, k half) are fenced from each other so that every
@@ -213,7 +186,7 @@ __global__ __launch_bounds__(kWave* WM, WM == 8 ? 1 : 2) void linear_kernel(cons
 #pragma unroll
       for (int t = 0; t < 6; ++t)
         acc[r / 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            w[r & 1][kW[t]], __builtin_bit_cast(bf16x8, xl[CUR][r & 1][kX[t]]), acc[r / 2], 0, 0, 0);
+            w[r & 1][kLimbA[t]], __builtin_bit_cast(bf16x8, xl[CUR][r & 1][kLimbB[t]]), acc[r / 2], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (!LAST) __syncthreads();

@@ -1,4 +1,5 @@
-// Paged causal prefill / chunked-prefill attention for gfx950 on fp32 MFMA.
+// Paged causal prefill / chunked-prefill attention for gfx950 on fp32 MFMA (and, for launches with
+// many query rows, prefill_wide.h's kernel on the bf16 matrix cores: use_wide below).
 //
 // One workgroup per (16-query tile, head, sequence); its KS waves split the
 // tile's keys (wave w takes key tiles w, w + KS, ...) and merge their partial
@@ -42,81 +43,14 @@
 #include <algorithm>
 
 #include "decode_wave.h"
+#include "prefill_args.h"
+#include "prefill_wide.h"
 #include "tq_internal.h"
 
 namespace tq {
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-
-constexpr int kTile = 16;  // queries per wave, keys per step
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kSlack = 8.f;  // log2 units a stale running maximum may trail a score by
-
-struct PrefillArgs {
-  float* out;
-  int64_t out_stride;
-  const float* q;
-  int64_t q_stride;
-  const float* pool_layer;
-  int64_t block_stride;
-  int64_t kv_stride;
-  int64_t head_stride;
-  const int32_t* block_tables;
-  int64_t bt_stride;
-  const int32_t* cu_q;
-  const int32_t* q_start;
-  const int32_t* seq_order;  // dispatch rank -> sequence, or nullptr for the natural order
-  int32_t* d_error;
-  float scale;
-  int32_t num_blocks;
-  int32_t num_heads;
-  int32_t block_size;
-  int32_t max_blocks;
-  int32_t num_q_rows;
-  int32_t qtiles;     // query tiles per (sequence, head): ceil(max_query_len / 16)
-  int32_t num_seqs;
-  int32_t groups;     // num_heads * num_seqs
-  int32_t total;      // workgroups: 8 XCDs x the most groups on one XCD x qtiles
-};
-
-constexpr int kXcds = 8;      // MI355X: workgroup i is dispatched to XCD i % 8
-// Word 3 of a raw (untyped) buffer descriptor on gfx9-family GPUs: data format 32 bits (a
-// nonzero format makes the loads valid), no swizzle, no typed conversion.
-constexpr int kBufferWord3 = 0x00020000;
-constexpr int kRound = 64;    // dispatches per XCD taken as one round (two per CU of its 32)
-
-// Maps the dispatch index to a work tile. Workgroup p runs on XCD p % 8 (checked
-// on MI355X with the XCC_ID register), and the XCD hands its workgroups to its 32
-// CUs round robin. The (sequence, head) groups are dealt out whole, group g to XCD
-// g % 8, so all query tiles of a group share one L2 for their K/V reads and the
-// heads of a long sequence spread over all eight XCDs; an XCD with one group fewer
-// than the most gets padding workgroups that exit at once. Inside an XCD the tiles
-// go out by cost (query tile index, descending across its G groups) and the rounds
-// of kRound dispatches snake: round k even takes cost ranks k kRound .. k kRound +
-// kRound - 1 in order, odd in reverse, so the tiles a CU receives over two rounds
-// add up to about the same number of key tiles (measured on 256-token chunks of 4
-// prompts: 15.1 / 24.9 / 34.5 -> 11.5 / 21.5 / 31.4 us at starts 0 / 256 / 512
-// against contiguous runs with the last query tiles first; rounds of 32 or 128 do
-// about as well, 16 worse; dealing contiguous runs of groups instead of every
-// eighth group left a 3-prompt chunk with one long prompt 45 % slower). Returns
-// false for a padding workgroup. `p` is the workgroup's index among the launch's prefill
-// workgroups, a multiple of 8 dispatches after the first (so p % 8 is still its XCD). The
-// sequence b it returns is a dispatch rank; a.seq_order maps it to the sequence itself.
-__device__ __forceinline__ bool tile_of(const PrefillArgs& a, int p, int& qt, int& h, int& b) {
-  const int xcd = p % kXcds, local = p / kXcds;
-  const int G = (a.groups - xcd + kXcds - 1) / kXcds;  // groups xcd, xcd + 8, ... on this XCD
-  const int n = G * a.qtiles;
-  if (local >= n) return false;
-  const int k = local / kRound, c = local - k * kRound;
-  const int m = min(kRound, n - k * kRound);  // size of this round
-  const int rank = k * kRound + ((k & 1) ? m - 1 - c : c);
-  qt = a.qtiles - 1 - rank / G;
-  const int seq_head = xcd + kXcds * (rank % G);
-  h = seq_head % a.num_heads;
-  b = seq_head / a.num_heads;
-  return true;
-}
 
 // Pointer to the first element of position `key` of this head's K tile (V is + kv_stride),
 // or nullptr when the block id is out of range.
@@ -161,11 +95,6 @@ __device__ __forceinline__ void load_kv_tile(const PrefillArgs& a, const int32_t
     vreg[s] = p != nullptr ? *reinterpret_cast<const float4*>(p + a.kv_stride + 4 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
   }
 }
-
-// Maxima are IEEE maximum (v_maximum3_f32 / v_maximum_f32): unlike fmaxf they need no
-// canonicalization of their operands, and a NaN score propagates instead of being dropped.
-__device__ __forceinline__ float max2(float a, float b) { return __builtin_elementwise_maximum(a, b); }
-__device__ __forceinline__ float max4(float a, float b, float c, float d) { return max2(max2(a, b), max2(c, d)); }
 
 // Max of v over the four lanes j, j + 16, j + 32, j + 48 (one query's lane groups), left in all
 // four: gfx950's cross-row lane swaps (v_permlane16_swap / v_permlane32_swap) on the VALU instead
@@ -596,6 +525,41 @@ constexpr int64_t kTwoTileMinTiles = 8192;
 // longest first (each XCD's share of the heavy sequences, then the rounds' mix) ran 3-16 %
 // faster on six draws of 32 prompts U[256,1024]. Key-split launches hold every workgroup at
 // once and keep the natural order.
+template <int BS>
+void launch_prefill_wide(const PrefillArgs& a_in, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
+  PrefillArgs a = a_in;
+  a.qtiles = (a.max_query_len + kWideRows - 1) / kWideRows;
+  a.total = kXcds * ((a.groups + kXcds - 1) / kXcds) * a.qtiles;
+  if (start == nullptr && stop == nullptr)
+    hipLaunchKernelGGL((prefill_wide_kernel<BS>), dim3((unsigned)a.total), dim3(kWave * kWideWaves), 0, stream, a);
+  else
+    hipExtLaunchKernelGGL((prefill_wide_kernel<BS>), dim3((unsigned)a.total), dim3(kWave * kWideWaves), 0, stream,
+                          start, stop, 0, a);
+}
+
+// Whether a launch runs on the 128-query workgroups of prefill_wide.h: block size 16 or 32, and of
+// the launches that would get one wave per 16-row tile (the key splits above fill the GPU better
+// with less work) those
+//  * whose workgroups are well filled: the query rows at least 0.4 of what the grid holds;
+//  * with contexts that amortise a workgroup's start: a table for 256 keys at block size 16, where
+//    the 16-row kernels are tuned, 128 at 32, where they look every key's block up;
+//  * at block size 16, with 1,280 waves of rows (2.5 workgroups for every 2 a CU holds at 4 waves).
+// Measured us (12 heads; 16-row kernels -> 128-query workgroups), block size 16: 32 prompts of
+// 256-1,023 rows 214 -> 172, 4 x 750-1,000 73 -> 53, 16 x 225-300 34 -> 29, 64 x 75-100 rows behind 200
+// keys 67 -> 47, 2 x 8,192 1,560 -> 1,026 (201 TFLOP/s); left out: 32 x 96-128 18.5 -> 20.0, 64 x 48-64
+// 14.7 -> 18.8, 7 prompts of 33-511 rows 26.5 -> 28.2, 2 x 1,000 45.7 -> 51.0, 200 x 15-20 behind 100 keys
+// 41 -> 55. Block size 32: 32 prompts of 256-1,023 rows 359 -> 173, 13 of 17-255 37 -> 19, 32 x 96-128
+// 29.6 -> 19.9; left out: 128 x 48-64 28.6 -> 31.6, 100 x 30-40 17.4 -> 23.9.
+bool use_wide(const PrefillArgs& a) {
+  if (a.block_size != 16 && a.block_size != 32) return false;
+  if (choose_key_split((int64_t)a.groups * a.qtiles) != 1) return false;
+  const int64_t head_rows = (int64_t)a.num_heads * a.num_q_rows;
+  const int64_t held = (int64_t)a.groups * ((a.max_query_len + kWideRows - 1) / kWideRows) * kWideRows;
+  const int64_t max_keys = (int64_t)a.max_blocks * a.block_size;
+  if (5 * head_rows < 2 * held) return false;
+  return a.block_size == 16 ? max_keys >= 256 && head_rows >= 1280 * 32 : max_keys >= 128;
+}
+
 template <int BS_CT>
 void launch_prefill(const PrefillArgs& a_in, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
   const int ks = choose_key_split((int64_t)a_in.groups * a_in.qtiles);
@@ -688,6 +652,7 @@ tq_status make_prefill_args(const PrefillCall& c, PrefillArgs& a, bool& empty) {
   a.max_blocks = c.max_blocks_per_seq;
   a.num_q_rows = c.num_q_rows;
   a.qtiles = (int32_t)qtiles;
+  a.max_query_len = c.max_query_len;
   a.num_seqs = c.num_seqs;
   const int64_t groups = (int64_t)c.num_heads * c.num_seqs;
   a.groups = (int32_t)groups;
@@ -796,6 +761,11 @@ extern "C" tq_status tq_paged_prefill(float* out, int64_t out_row_stride, const 
                                          a, empty);
   if (st != TQ_OK || empty) return st;
   hipStream_t s = (hipStream_t)stream;
+  if (use_wide(a)) {
+    if (block_size == 16) launch_prefill_wide<16>(a, s, timing.start, timing.stop);
+    else launch_prefill_wide<32>(a, s, timing.start, timing.stop);
+    return check_launch();
+  }
   switch (block_size) {
     case 16: launch_prefill<16>(a, s, timing.start, timing.stop); break;
     default: launch_prefill<0>(a, s, timing.start, timing.stop); break;
@@ -812,8 +782,11 @@ extern "C" size_t tq_paged_mixed_workspace_size(int32_t num_decode_seqs, int32_t
   if (num_decode_seqs <= 0 || num_heads <= 0 || head_dim != kHeadDim || max_context_len <= 0) return 0;
   if (partition_tokens < 0 || partition_tokens % kChunk != 0 || partition_tokens > kMaxPartition) return 0;
   const int ks = prefill_key_split(num_prefill_seqs, num_heads, max_query_len);
-  return decode_workspace_bytes(num_decode_seqs, num_heads,
-                                decode_grid(num_decode_seqs, num_heads, max_context_len, partition_tokens, ks));
+  // Enough for either form of the call (one grid, or the decode launch and the wide prefill).
+  return std::max(decode_workspace_bytes(num_decode_seqs, num_heads,
+                                         decode_grid(num_decode_seqs, num_heads, max_context_len, partition_tokens, ks)),
+                  tq_paged_decode_workspace_size(num_decode_seqs, num_heads, head_dim, max_context_len,
+                                                 partition_tokens));
 }
 
 extern "C" tq_status tq_paged_mixed(float* dec_out, int64_t dec_out_row_stride, const float* dec_q,
@@ -858,6 +831,21 @@ extern "C" tq_status tq_paged_mixed(float* dec_out, int64_t dec_out_row_stride, 
                                     nullptr, num_prefill_seqs, num_q_rows, max_query_len, scale, d_error},
                                    pa, empty);
   if (st != TQ_OK) return st;
+  if (use_wide(pa)) {
+    // Many prefill rows: their own launch on the bf16 matrix cores saves more of them (a tenth to a
+    // third, more at block size 32: use_wide) than the shared grid hides of a step (6 % of one with 1,024
+    // prefill rows beside 128 decoding sequences).
+    tq_set_timing_events(timing.start, nullptr);
+    st = tq_paged_decode_write(dec_out, dec_out_row_stride, dec_q, dec_q_row_stride, k_new, k_new_row_stride, v_new,
+                               v_new_row_stride, pool, num_blocks, num_layers, num_heads, block_size, head_dim, layer,
+                               dec_block_tables, dec_block_table_stride, dec_max_blocks_per_seq, context_lens,
+                               seq_order, num_decode_seqs, max_context_len, scale, partition_tokens, workspace,
+                               workspace_bytes, d_error, stream);
+    if (st != TQ_OK) return st;
+    if (block_size == 16) launch_prefill_wide<16>(pa, (hipStream_t)stream, nullptr, timing.stop);
+    else launch_prefill_wide<32>(pa, (hipStream_t)stream, nullptr, timing.stop);
+    return check_launch();
+  }
   const int ks = choose_key_split((int64_t)pa.groups * pa.qtiles);
   DecodeArgs da;
   st = make_decode_args({dec_out, dec_out_row_stride, dec_q, dec_q_row_stride, k_new, k_new_row_stride, v_new,
