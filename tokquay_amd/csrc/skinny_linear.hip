@@ -147,13 +147,25 @@ __global__ __launch_bounds__(kWave* KW) void skinny_linear_kernel(const SkinnyAr
     }
   }
 
-  // W rows n_base + 16 r + i; rows past N (the ragged last block) read row N - 1 and are not
-  // stored.
+  // W rows n_base + 16 r + i; rows past N (the ragged last block) read row N - 1 and are not stored.
+  // The MFMA wants row lane % 16, chunk (float4) lane / 16 of each 16-wide k block. With a row of its
+  // own per lane the address unit takes one lane a clock (16 B); with four lanes a row four. So
+  // kCoalesced launches load row lane / 4, chunk lane % 4, and operand() moves the lanes into place
+  // through the LDS crossbar. It pays where a CU streams enough weights: 8 rows, weights evicted,
+  // the LM head 41.0 -> 37.9 us (with argmax 44.7 -> 39.6), 64 rows 13.3 / 7.3 / 13.8 / 14.1 -> 13.0 / 6.9 /
+  // 13.5 / 12.7 for the four projections; c_attn and c_fc with the LayerNorm and the split mlp.c_proj
+  // at up to 16 rows are bound by latency and lost 1-2 %.
+  constexpr bool kCoalesced = R > 1 || MB > 1 || (!LN && KSPLIT == 1);
+  const int w_row = kCoalesced ? lane >> 2 : i, w_chunk = kCoalesced ? lane & 3 : g;
   auto load_w = [&](floatx4 (&wv)[T], int r) {
-    const int n = min(n_base + 16 * r + i, a.N - 1);
-    const float* wp = a.w + (int64_t)n * a.K + k_lo + 4 * g;
+    const int n = min(n_base + 16 * r + w_row, a.N - 1);
+    const float* wp = a.w + (int64_t)n * a.K + k_lo + 4 * w_chunk;
 #pragma unroll
     for (int t = 0; t < T; ++t) wv[t] = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(wp + 16 * t));
+  };
+  const int from = 4 * (4 * i + g);  // byte address of the lane that loaded (row i, chunk g)
+  auto operand = [&](float v) {
+    return kCoalesced ? __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(v))) : v;
   };
   floatx4 wb[R > 1 ? 2 : 1][T];
   load_w(wb[0], 0);
@@ -223,7 +235,11 @@ __global__ __launch_bounds__(kWave* KW) void skinny_linear_kernel(const SkinnyAr
     const int n_cur = cb_cur * (16 * R);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const floatx4(&wv)[T] = wb[r & 1];
+      floatx4 wv[T];
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) wv[t][c] = operand(wb[r & 1][t][c]);
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) acc[r][mb] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
