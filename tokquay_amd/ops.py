@@ -586,12 +586,12 @@ def linear(x: torch.Tensor, layer: torch.nn.Linear, gelu: bool = False) -> torch
     """``x @ layer.weight.T + layer.bias`` (then the tanh GELU when ``gelu``): ``tq_linear`` over many
     rows (``uses_rows_kernel``), else hipBLASLt in the weight layout ``GEMM_NN_SHAPES`` names for
     this shape. On the CPU: torch's ``F.linear`` and the tanh GELU."""
+    weight, bias = layer.weight, layer.bias  # each a Module lookup: once
     if not x.is_cuda:
-        y = torch.nn.functional.linear(x, layer.weight, layer.bias)
+        y = torch.nn.functional.linear(x, weight, bias)
         return torch.nn.functional.gelu(y, approximate="tanh") if gelu else y
-    if _rows_kernel_takes(x, layer.weight, layer.bias):
-        return _rows_linear(x, layer.weight, layer.bias, gelu)
-    out_f, in_f = layer.weight.shape
+    if _rows_kernel_takes(x, weight, bias):
+        return _rows_linear(x, weight, bias, gelu)
+    out_f, in_f = weight.shape
     nn_layout = uses_nn_layout(x.shape[0], out_f, in_f, gelu)
-    w = transposed_weight(layer) if nn_layout else layer.weight.t()
-    return _gemm(x, w, layer.bias, gelu)
+    return _gemm(x, transposed_weight(layer) if nn_layout else weight.t(), bias, gelu)
