@@ -27,7 +27,7 @@
 // log2 e, so p = 2^(s - m) on v_exp_f32). The max is lazy: it moves, and the
 // accumulators are rescaled, only when a score passes it by more than 2^8.
 //
-// With block size 16 the key loop is software-pipelined: each wave issues the
+// With block size 16 or 32 the key loop is software-pipelined: each wave issues the
 // next key tile's K/V loads (buffer loads off descriptors on the block's K and V
 // tiles) before the current tile's math. The MFMA results stay in VGPRs (built
 // with -amdgpu-mfma-vgpr-form), so the per-tile rescale and the softmax read them
@@ -106,30 +106,41 @@ __device__ __forceinline__ float max_over_lane_groups(float v) {
   return max2(__uint_as_float(p32[0]), __uint_as_float(p32[1]));  // lanes 0-31 <-> 32-63
 }
 
-// Same loads when a 16-key tile is exactly one block (block size 16): the tile's block id arrives
-// as a wave-uniform scalar (blk < 0: out of range). They are buffer loads off two descriptors
-// built on the block's K and V tiles (scalar registers), with fixed per-lane byte offsets: lane
-// (j, g) reads K row j (dims 16g ..) and V rows 4g .. 4g + 3 (dims 4j ..), so no per-tile 64-bit
-// address arithmetic runs on the VALU. The descriptors' sizes do the masking: they cover the
-// tile's rows below kend (none for a bad block id), and the hardware returns zeros for every load
-// past them, which is what the keys past the range and a bad block must contribute.
+// Same loads when a 16-key tile lies in one block (block size 16 or 32): the tile's block id arrives
+// as a wave-uniform scalar (blk < 0: out of range). They are buffer loads off two descriptors built
+// on the tile's K and V rows (scalar registers), with fixed per-lane byte offsets, so no per-tile
+// 64-bit address arithmetic runs on the VALU. The descriptors' sizes do the masking: they cover
+// the tile's rows below kend (none for a bad block id), and the hardware returns zeros for every
+// load past them, which is what the keys past the range and a bad block must contribute.
+//
+// V row 4 g + s, dims 4 j .. goes to vreg[s] (a load covers four whole rows). The QK product wants a K row
+// per lane, dims 16 g ..; loaded that way the address unit takes one lane a clock, 256 clocks of the
+// 320 a key tile's loads take it, and with 3 workgroups of 4 waves per CU that is what bound the
+// 256-token chunks. ROWS loads K in address order instead (kreg[4 t ..]: row 4 t + g, dims 4 j ..), and
+// place_k() gets the rows into place through LDS. The launches with one pipelined wave per tile keep
+// the direct loads: there the registers place_k() takes cost a wave per SIMD. Measured us (direct ->
+// place_k()): 4 chunks of 256 rows at 0 / 256 / 512 10.5 / 18.7 / 27.0 -> 10.2 / 18.2 / 25.5, 8 x 256 behind
+// 700 keys 64.7 -> 58.2, a mixed launch of 4 x 250-256 rows at 512 beside 128 decode rows 71.6 -> 64.6;
+// one wave per tile: 7 prompts of 33-511 rows 26.7 -> 28.0, two tiles per wave 44.0 -> 50.0.
+template <int BS, bool ROWS>
 __device__ __forceinline__ void load_kv_block_tile(const PrefillArgs& a, const float* head_base, int32_t blk,
                                                    int kt, int kend, int j, int g, float (&kreg)[16],
                                                    float4 (&vreg)[4]) {
   constexpr int kRowBytes = kHeadDim * 4;
-  const uint32_t k_off = (uint32_t)(j * kHeadDim + 16 * g) * 4u;
+  const uint32_t k_off = ROWS ? (uint32_t)(g * kHeadDim + 4 * j) * 4u : (uint32_t)(j * kHeadDim + 16 * g) * 4u;
+  constexpr uint32_t kKStep = ROWS ? 4 * kRowBytes : 16;
   const uint32_t v_off = (uint32_t)(4 * g * kHeadDim + 4 * j) * 4u;
   const int rows = blk < 0 ? 0 : min(kTile, kend - kt);  // uniform: rows that count
-  const float* kb = head_base + (int64_t)(blk < 0 ? 0 : blk) * a.block_stride;
+  const float* kb = head_base + (int64_t)(blk < 0 ? 0 : blk) * a.block_stride + (BS == kTile ? 0 : kt % BS * kHeadDim);
   const __amdgpu_buffer_rsrc_t kd =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kb), (short)0, rows * kRowBytes, kBufferWord3);
   const __amdgpu_buffer_rsrc_t vd = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kb + a.kv_stride),
                                                                       (short)0, rows * kRowBytes, kBufferWord3);
 #pragma unroll
-  for (int v4 = 0; v4 < 4; ++v4) {
-    const auto x = __builtin_amdgcn_raw_buffer_load_b128(kd, k_off + 16u * v4, 0, 0);
+  for (int t = 0; t < 4; ++t) {
+    const auto x = __builtin_amdgcn_raw_buffer_load_b128(kd, k_off + (uint32_t)t * kKStep, 0, 0);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) kreg[4 * v4 + c] = __uint_as_float(x[c]);
+    for (int c = 0; c < 4; ++c) kreg[4 * t + c] = __uint_as_float(x[c]);
   }
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
@@ -138,16 +149,36 @@ __device__ __forceinline__ void load_kv_block_tile(const PrefillArgs& a, const f
   }
 }
 
+// Moves a K tile loaded with ROWS to the QK product's A operand, through the wave's own
+// 4 KiB of LDS: kout[s] of lane (j, g) = K[row j][16 g + s]. Float4 c of row r sits in slot 16 r + (c ^ r):
+// neither side has bank conflicts.
+__device__ __forceinline__ void place_k(float4* slots, int j, int g, const float (&kreg)[16], float (&kout)[16]) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int r = 4 * t + g;
+    slots[16 * r + (j ^ r)] = make_float4(kreg[4 * t], kreg[4 * t + 1], kreg[4 * t + 2], kreg[4 * t + 3]);
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const float4 x = slots[16 * j + ((4 * g + v) ^ j)];
+    kout[4 * v + 0] = x.x;
+    kout[4 * v + 1] = x.y;
+    kout[4 * v + 2] = x.z;
+    kout[4 * v + 3] = x.w;
+  }
+}
+
 // The work of prefill workgroup `dispatch` (its KS waves): QH consecutive query tiles of one head
 // of one sequence, or nothing for a padding workgroup. QH = 2 (one wave per workgroup only) feeds
 // each key tile's loads to twice the MFMAs and gives the wave two independent softmax chains.
-// PIPE: the software-pipelined key loop (block size 16 only). The mixed launch keeps the plain
+// PIPE: the software-pipelined key loop (block sizes 16 and 32). The mixed launch keeps the plain
 // loop: with the pipelined one (126 VGPRs, its decode workgroups still at 4 waves per SIMD) the
 // steps of four 256-token prompt chunks beside 128 decoding sequences ran from 3 % faster to 2 %
 // slower depending on the chunk.
-template <int BS_CT, int KS, int QH = 1, bool PIPE = (BS_CT == kTile)>
+template <int BS_CT, int KS, int QH = 1, bool PIPE = (BS_CT > 0)>
 __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int dispatch) {
-  static_assert(!PIPE || BS_CT == kTile, "the pipelined key loop reads one block per key tile");
+  static_assert(BS_CT == 0 || BS_CT % kTile == 0, "a key tile lies in one block");
+  static_assert(!PIPE || BS_CT > 0, "the pipelined key loop reads one block per key tile");
   static_assert(QH == 1 || KS == 1, "two query tiles per wave only without a key split");
   const int lane = threadIdx.x & (kWave - 1);
   // Wave-uniform by construction; readfirstlane lets the compiler keep the key-tile loop
@@ -263,7 +294,16 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
   // running-maximum test on each lane's own four scores (the lane-group maximum only when some
   // lane's test fires), max as v_maximum3_f32 (no operand canonicalization), and one ballot
   // for all of the wave's query tiles.
-  auto consume = [&](int kt, const float (&kreg)[16], const float4 (&vreg)[4]) {
+  constexpr bool kPlaceK = BS_CT > 0 && (KS > 1 || !PIPE);
+  __shared__ float4 s_k[KS][kPlaceK ? kTile * kHeadDim / 4 : 1];
+  auto consume = [&](int kt, const float (&kload)[16], const float4 (&vreg)[4]) {
+      float kreg[16];
+      if constexpr (kPlaceK) {
+        place_k(s_k[wave], j, g, kload, kreg);
+      } else {
+  #pragma unroll
+        for (int s = 0; s < 16; ++s) kreg[s] = kload[s];
+      }
       floatx4 st[QH];
   #pragma unroll
       for (int u = 0; u < QH; ++u) st[u] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -326,8 +366,7 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
   };
 
   if constexpr (PIPE) {
-    // Block size 16: tile i is block table entry i.
-    // The ids of 64 consecutive tiles are held one per lane and fetched per tile with
+    // The ids of 64 consecutive blocks are held one per lane and fetched per tile with
     // v_readlane (no table loads in the loop); the lane copy is refreshed when the
     // wave moves to the next 64.
     // The loop is software-pipelined over two register buffers: the next tile's
@@ -335,10 +374,10 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
     int tb_base = -1;
     int32_t tb_id = 0;
     auto fetch = [&](int kt, float (&kreg)[16], float4 (&vreg)[4]) {
-      const int ti = kt / kTile;
+      const int ti = kt / BS_CT;
       if ((ti & ~63) != tb_base) {  // wave-uniform
         tb_base = ti & ~63;
-        const int nblk = (kend + kTile - 1) / kTile;
+        const int nblk = (kend + BS_CT - 1) / BS_CT;
         tb_id = -1;
         if (tb_base + lane < nblk) {
           const int32_t id = bt[tb_base + lane];
@@ -346,7 +385,7 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
           else flag_error(a.d_error, TQ_DEVERR_BLOCK_ID);
         }
       }
-      load_kv_block_tile(a, head_base, __builtin_amdgcn_readlane(tb_id, ti - tb_base), kt, kend, j, g, kreg, vreg);
+      load_kv_block_tile<BS_CT, kPlaceK>(a, head_base, __builtin_amdgcn_readlane(tb_id, ti - tb_base), kt, kend, j, g, kreg, vreg);
     };
     const int step = KS * kTile;
     int kt = wave * kTile;
@@ -396,11 +435,11 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
     for (int kt = wave * kTile; kt < kend; kt += KS * kTile) {
       float kreg[16];
       float4 vreg[4];
-      if constexpr (BS_CT == kTile) {
-        const int ti = kt / kTile;
+      if constexpr (BS_CT > 0) {
+        const int ti = kt / BS_CT;
         if ((ti & ~63) != tb_base) {  // wave-uniform
           tb_base = ti & ~63;
-          const int nblk = (kend + kTile - 1) / kTile;
+          const int nblk = (kend + BS_CT - 1) / BS_CT;
           tb_id = -1;
           if (tb_base + lane < nblk) {
             const int32_t id = bt[tb_base + lane];
@@ -408,7 +447,7 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
             else flag_error(a.d_error, TQ_DEVERR_BLOCK_ID);
           }
         }
-        load_kv_block_tile(a, head_base, __builtin_amdgcn_readlane(tb_id, ti - tb_base), kt, kend, j, g, kreg, vreg);
+        load_kv_block_tile<BS_CT, kPlaceK>(a, head_base, __builtin_amdgcn_readlane(tb_id, ti - tb_base), kt, kend, j, g, kreg, vreg);
       } else {
         load_kv_tile<BS_CT>(a, bt, head_base, bs, kt, kend, j, g, kreg, vreg);
       }
@@ -541,23 +580,19 @@ void launch_prefill_wide(const PrefillArgs& a_in, hipStream_t stream, hipEvent_t
 // the launches that would get one wave per 16-row tile (the key splits above fill the GPU better
 // with less work) those
 //  * whose workgroups are well filled: the query rows at least 0.4 of what the grid holds;
-//  * with contexts that amortise a workgroup's start: a table for 256 keys at block size 16, where
-//    the 16-row kernels are tuned, 128 at 32, where they look every key's block up;
-//  * at block size 16, with 1,280 waves of rows (2.5 workgroups for every 2 a CU holds at 4 waves).
+//  * whose tables have room for 256 keys, to amortise a workgroup's start;
+//  * with 1,280 waves of rows (2.5 workgroups for every 2 a CU holds, at 4 waves).
 // Measured us (12 heads; 16-row kernels -> 128-query workgroups), block size 16: 32 prompts of
 // 256-1,023 rows 214 -> 172, 4 x 750-1,000 73 -> 53, 16 x 225-300 34 -> 29, 64 x 75-100 rows behind 200
 // keys 67 -> 47, 2 x 8,192 1,560 -> 1,026 (201 TFLOP/s); left out: 32 x 96-128 18.5 -> 20.0, 64 x 48-64
 // 14.7 -> 18.8, 7 prompts of 33-511 rows 26.5 -> 28.2, 2 x 1,000 45.7 -> 51.0, 200 x 15-20 behind 100 keys
-// 41 -> 55. Block size 32: 32 prompts of 256-1,023 rows 359 -> 173, 13 of 17-255 37 -> 19, 32 x 96-128
-// 29.6 -> 19.9; left out: 128 x 48-64 28.6 -> 31.6, 100 x 30-40 17.4 -> 23.9.
+// 41 -> 55. Block size 32 takes the same times.
 bool use_wide(const PrefillArgs& a) {
   if (a.block_size != 16 && a.block_size != 32) return false;
   if (choose_key_split((int64_t)a.groups * a.qtiles) != 1) return false;
   const int64_t head_rows = (int64_t)a.num_heads * a.num_q_rows;
   const int64_t held = (int64_t)a.groups * ((a.max_query_len + kWideRows - 1) / kWideRows) * kWideRows;
-  const int64_t max_keys = (int64_t)a.max_blocks * a.block_size;
-  if (5 * head_rows < 2 * held) return false;
-  return a.block_size == 16 ? max_keys >= 256 && head_rows >= 1280 * 32 : max_keys >= 128;
+  return head_rows >= 1280 * 32 && 5 * head_rows >= 2 * held && (int64_t)a.max_blocks * a.block_size >= 256;
 }
 
 template <int BS_CT>
@@ -567,7 +602,7 @@ void launch_prefill(const PrefillArgs& a_in, hipStream_t stream, hipEvent_t star
   if (ks != 1) a.seq_order = nullptr;
   switch (ks) {
     case 1:
-      if (BS_CT == kTile && (int64_t)a.num_heads * ((a.num_q_rows + kTile - 1) / kTile) >= kTwoTileMinTiles) {
+      if (BS_CT > 0 && (int64_t)a.num_heads * ((a.num_q_rows + kTile - 1) / kTile) >= kTwoTileMinTiles) {
         // More tiles than the key split pays for, and many rows: with block size 16 each wave
         // takes two consecutive query tiles, so every key tile's loads feed both and the wave has
         // two independent softmax chains (per launch: 32 prompts U[256,1024] 248 -> 233 us,
@@ -576,7 +611,7 @@ void launch_prefill(const PrefillArgs& a_in, hipStream_t stream, hipEvent_t star
         PrefillArgs a2 = a;
         a2.qtiles = (a.qtiles + 1) / 2;
         a2.total = kXcds * ((a.groups + kXcds - 1) / kXcds) * a2.qtiles;
-        if constexpr (BS_CT == kTile) launch_prefill_ks<BS_CT, 1, 2>(a2, stream, start, stop);
+        if constexpr (BS_CT > 0) launch_prefill_ks<BS_CT, 1, 2>(a2, stream, start, stop);
       } else {
         launch_prefill_ks<BS_CT, 1>(a, stream, start, stop);
       }
@@ -768,6 +803,7 @@ extern "C" tq_status tq_paged_prefill(float* out, int64_t out_row_stride, const 
   }
   switch (block_size) {
     case 16: launch_prefill<16>(a, s, timing.start, timing.stop); break;
+    case 32: launch_prefill<32>(a, s, timing.start, timing.stop); break;
     default: launch_prefill<0>(a, s, timing.start, timing.stop); break;
   }
   return check_launch();
@@ -833,7 +869,7 @@ extern "C" tq_status tq_paged_mixed(float* dec_out, int64_t dec_out_row_stride, 
   if (st != TQ_OK) return st;
   if (use_wide(pa)) {
     // Many prefill rows: their own launch on the bf16 matrix cores saves more of them (a tenth to a
-    // third, more at block size 32: use_wide) than the shared grid hides of a step (6 % of one with 1,024
+    // third: use_wide) than the shared grid hides of a step (6 % of one with 1,024
     // prefill rows beside 128 decoding sequences).
     tq_set_timing_events(timing.start, nullptr);
     st = tq_paged_decode_write(dec_out, dec_out_row_stride, dec_q, dec_q_row_stride, k_new, k_new_row_stride, v_new,
@@ -867,7 +903,7 @@ extern "C" tq_status tq_paged_mixed(float* dec_out, int64_t dec_out_row_stride, 
   hipEvent_t stop = merge ? nullptr : timing.stop;
   switch (block_size) {
     case 16: launch_mixed<16, 16>(pa, da, ks, g32, u32, s, timing.start, stop); break;
-    case 32: launch_mixed<32, 0>(pa, da, ks, g32, u32, s, timing.start, stop); break;
+    case 32: launch_mixed<32, 32>(pa, da, ks, g32, u32, s, timing.start, stop); break;
     default: launch_mixed<0, 0>(pa, da, ks, g32, u32, s, timing.start, stop); break;
   }
   if (merge) launch_decode_merge(da, num_decode_seqs, s, timing.stop);
