@@ -354,7 +354,12 @@ tq_status tq_argmax_rows(int64_t* out, const float* logits, int64_t num_rows, in
  */
 tq_status tq_linear(float* y, int64_t y_stride, const float* x, int64_t x_stride, int32_t M,
                     const float* w, const float* bias, int32_t N, int32_t K,
-                    int32_t epilogue, void* stream);
+                    int32_t epilogue, void* workspace, size_t workspace_bytes, void* stream);
+
+/* Bytes of workspace tq_linear needs for these sizes (0 for most: only outputs of too few tiles
+ * to fill the GPU are computed in parts of K). 16-byte aligned; its contents need not start at
+ * zero. A call whose y or bias is not 16-byte aligned uses none. */
+size_t tq_linear_workspace_size(int32_t M, int32_t N, int32_t K);
 
 /*
  * Residual add + LayerNorm over rows of `cols` fp32 values:

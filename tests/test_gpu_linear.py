@@ -10,7 +10,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from tokquay_amd import ops
+from tokquay_amd import _lib, ops
 
 EPS = 2.0**-24
 
@@ -41,6 +41,8 @@ def _inputs(m, n, k, bias=True, seed=0):
     (1, 1, 32), (1, 33, 64), (31, 64, 96), (33, 50, 768), (127, 96, 32), (129, 127, 64), (255, 2304, 768),
     (257, 770, 96), (640, 2304, 768), (1000, 2304, 768), (1100, 3072, 64), (1987, 2304, 768), (2048, 3072, 96),
     (2100, 768, 3072), (4097, 1024, 32), (66, 50257, 768),
+    # K in parts: 2, 3, 4, 6, 10 and 16 of them, ragged rows and columns
+    (70, 100, 256), (129, 516, 384), (640, 768, 3072), (321, 768, 3072), (130, 1600, 1600), (100, 768, 3072),
 ])  # fmt: skip
 @pytest.mark.parametrize("gelu", [False, True])
 def test_linear_matches_float64(m, n, k, gelu):
@@ -85,8 +87,31 @@ def test_non_finite_inputs_follow_fp32():
     torch.testing.assert_close(got[fin], ref[fin], rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.gpu
+def test_parts_of_k_follow_fp32_and_need_their_workspace():
+    x, w, b = _inputs(130, 512, 1024)
+    x[5, 700], w[9, 3] = float("inf"), float("nan")
+    got = ops._rows_linear(x, w, b, True)
+    ref = torch.nn.functional.gelu(torch.addmm(b.double(), x.double(), w.double().t()), approximate="tanh").float()
+    assert torch.equal(got.isnan(), ref.isnan())
+    fin = ref.isfinite()
+    torch.testing.assert_close(got[fin], ref[fin], rtol=1e-4, atol=1e-4)
+    L = _lib.lib()
+    assert L.tq_linear_workspace_size(130, 512, 1024) == 8 * 130 * 512 * 4
+    y = torch.empty(130, 512, device="cuda")
+    args = (y.data_ptr(), 512, x.data_ptr(), 1024, 130, w.data_ptr(), b.data_ptr(), 512, 1024, 0)
+    assert L.tq_linear(*args, None, 0, 0) == 3
+    assert L.tq_linear(*args, y.data_ptr(), 8 * 130 * 512 * 4 - 1, 0) == 3
+
+
 def test_rule():
-    """Few tiles, K not in whole steps: the library; many: tq_linear."""
+    """Few tiles, K not in whole steps: the library; many, or long K to split: tq_linear."""
+    assert ops.uses_rows_kernel(320, 768, 3072) and not ops.uses_rows_kernel(319, 768, 3072)
+    assert not ops.uses_rows_kernel(640, 768, 768) and not ops.uses_rows_kernel(640, 766, 3072)
+    assert not ops.uses_rows_kernel(1536, 768, 3072)  # 144 tiles: neither enough nor few enough for two parts
+    assert _lib.lib().tq_linear_workspace_size(1536, 768, 3072) == 0
+    assert _lib.lib().tq_linear_workspace_size(640, 766, 3072) == 0
+    assert _lib.lib().tq_linear_workspace_size(640, 768, 3072) == 4 * 640 * 768 * 4
     assert not ops.uses_rows_kernel(256, 2304, 768) and not ops.uses_rows_kernel(0, 2304, 768)
     assert ops.uses_rows_kernel(640, 2304, 768) and ops.uses_rows_kernel(2048, 768, 3072)
     assert ops.uses_rows_kernel(65, 50257, 768)

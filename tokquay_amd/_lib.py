@@ -144,9 +144,10 @@ SIGNATURES: dict[str, tuple] = {
         [
             c_f32p, ctypes.c_int64, c_f32p, ctypes.c_int64, ctypes.c_int32,  # y, y_stride, x, x_stride, M
             c_f32p, c_f32p, ctypes.c_int32, ctypes.c_int32,  # w, bias, N, K
-            ctypes.c_int32, ctypes.c_void_p,  # epilogue, stream
+            ctypes.c_int32, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p,  # epilogue, workspace, its bytes, stream
         ],
     ),
+    "tq_linear_workspace_size": (ctypes.c_size_t, [ctypes.c_int32] * 3),
     "tq_skinny_linear": (
         ctypes.c_int,
         [

@@ -37,6 +37,9 @@
 //    so neither side has bank conflicts.
 //  * A step's loads are issued two steps before they are split (one where the registers allow no
 //    more): weights come from HBM in a model's step, and one step is shorter than their latency.
+// Outputs of fewer than 160 tiles of 128 x 64 are computed in parts of K, a workgroup per tile and
+// part, and summed in order (with bias and epilogue) by a second launch: no tile waits for another
+// workgroup, and the partial sums live in the caller's workspace.
 // Measured (GPU time, MI355X, weights evicted between calls) against the library's fp32 GEMM: 1,987
 // rows, [N, K] = [2304, 768] / [3072, 768] / [768, 3072] / [768, 768]: 76 / 78 / 86 / 27 -> 45 / 51 /
 // 67 / 20 us; 8,192 rows (operands resident): 221 / 280 / 266 / 85 -> 154 / 191 / 181 / 54 us (188-213
@@ -69,7 +72,9 @@ struct LinearArgs {
   int32_t M, N, K;
   int32_t m_tiles, n_tiles;
   int32_t epilogue;
-  int32_t vec;  // rows of y and bias can be accessed four floats at a time
+  int32_t vec;       // rows of y and bias can be accessed four floats at a time
+  int32_t k_part;    // k a workgroup covers: K, or K / parts with blockIdx.y the part
+  int32_t parts;
 };
 
 // v (tanh-form GELU): v / (1 + exp(-2u)) = 0.5 v (1 + tanh u), u = sqrt(2/pi) (v + 0.044715 v^3),
@@ -115,13 +120,15 @@ __global__ __launch_bounds__(kWave* WM, WM == 8 ? 1 : 2) void linear_kernel(cons
   const int m_tile = rows_first ? lo : hi, n_tile = rows_first ? hi : lo;
   const int m0 = m_tile * BM + 32 * wave, n0 = n_tile * BN;
 
+  const int k_lo = blockIdx.y * a.k_part;
   // Descriptors on the wave's rows of X and the tile's rows of W: loads past the last row give 0.
   const int x_rows = max(0, min(32, a.M - m0)), w_rows = min(BN, a.N - n0);
   const __amdgpu_buffer_rsrc_t xd = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(a.x + (int64_t)min(m0, a.M - 1) * a.x_stride), (short)0,
-      x_rows > 0 ? (int32_t)(((x_rows - 1) * a.x_stride + a.K) * 4) : 0, kBufferWord3);
-  const __amdgpu_buffer_rsrc_t wd = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.w + (int64_t)n0 * a.K),
-                                                                      (short)0, w_rows * a.K * 4, kBufferWord3);
+      const_cast<float*>(a.x + (int64_t)min(m0, a.M - 1) * a.x_stride + k_lo), (short)0,
+      x_rows > 0 ? (int32_t)(((x_rows - 1) * a.x_stride + a.k_part) * 4) : 0, kBufferWord3);
+  const __amdgpu_buffer_rsrc_t wd =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.w + (int64_t)n0 * a.K + k_lo), (short)0,
+                                        ((w_rows - 1) * a.K + a.k_part) * 4, kBufferWord3);
   const uint32_t x_off = (uint32_t)(i * a.x_stride + 8 * g) * 4u;  // row i, octet g of each k half
   // Staging: unit rows lane / 4, k octet lane % 4 (k half octet / 2).
   const int sr = lane >> 2, so = lane & 3;
@@ -192,7 +199,7 @@ __global__ __launch_bounds__(kWave* WM, WM == 8 ? 1 : 2) void linear_kernel(cons
     if constexpr (!LAST) __syncthreads();
   };
 
-  const int steps = a.K / kStep;
+  const int steps = a.k_part / kStep;
   const int32_t k_end = (steps - 1) * kStep;
   auto load_step = [&](int at, int32_t k) {
 #pragma unroll
@@ -223,6 +230,8 @@ __global__ __launch_bounds__(kWave* WM, WM == 8 ? 1 : 2) void linear_kernel(cons
     step(Even{}, std::true_type{}, 0);
   }
 
+  // A part of K stores its plain partial sums (no bias, no epilogue) into its own [M, N] of y.
+  float* y = a.y + (int64_t)blockIdx.y * a.M * a.N;
   auto finish = [&](float v) { return a.epilogue == kEpiGelu ? gelu(v) : v; };
   float probe = 0.f;  // NaN once any accumulator is infinite or NaN
 #pragma unroll
@@ -235,11 +244,11 @@ __global__ __launch_bounds__(kWave* WM, WM == 8 ? 1 : 2) void linear_kernel(cons
     for (int e = lane; e < 32 * BN; e += kWave) {
       const int m = m0 + e / BN, c = n0 + e % BN;
       if (m >= a.M || c >= a.N) continue;
-      const float* xp = a.x + (int64_t)m * a.x_stride;
-      const float* wp = a.w + (int64_t)c * a.K;
+      const float* xp = a.x + (int64_t)m * a.x_stride + k_lo;
+      const float* wp = a.w + (int64_t)c * a.K + k_lo;
       float v = 0.f;
-      for (int k = 0; k < a.K; ++k) v = fmaf(xp[k], wp[k], v);
-      a.y[(int64_t)m * a.y_stride + c] = finish(a.bias != nullptr ? v + a.bias[c] : v);
+      for (int k = 0; k < a.k_part; ++k) v = fmaf(xp[k], wp[k], v);
+      y[(int64_t)m * a.y_stride + c] = finish(a.bias != nullptr ? v + a.bias[c] : v);
     }
     return;
   }
@@ -269,7 +278,7 @@ __global__ __launch_bounds__(kWave* WM, WM == 8 ? 1 : 2) void linear_kernel(cons
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = finish(v[e] + b[e]);
       if (m0 + row >= a.M) continue;
-      float* yp = a.y + (int64_t)(m0 + row) * a.y_stride + c;
+      float* yp = y + (int64_t)(m0 + row) * a.y_stride + c;
       if (a.vec) {
         if (c < a.N) *reinterpret_cast<floatx4*>(yp) = v;
       } else {
@@ -285,7 +294,38 @@ template <int WM, int NB, int DEPTH>
 void launch(LinearArgs a, hipStream_t s) {
   a.m_tiles = (a.M + 32 * WM - 1) / (32 * WM);
   a.n_tiles = (a.N + 32 * NB - 1) / (32 * NB);
-  hipLaunchKernelGGL((linear_kernel<WM, NB, DEPTH>), dim3((unsigned)(a.m_tiles * a.n_tiles)), dim3(kWave * WM), 0, s, a);
+  hipLaunchKernelGGL((linear_kernel<WM, NB, DEPTH>), dim3((unsigned)(a.m_tiles * a.n_tiles), (unsigned)a.parts),
+                     dim3(kWave * WM), 0, s, a);
+}
+
+// y = epilogue( the parts' sums, added in order, + bias ): a float4 per thread.
+__global__ __launch_bounds__(256) void linear_sum_kernel(const LinearArgs a, const float* partials) {
+  const int64_t at = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x), size = (int64_t)a.M * a.N;
+  if (at >= size) return;
+  floatx4 v = *reinterpret_cast<const floatx4*>(partials + at);
+#pragma unroll 4
+  for (int p = 1; p < a.parts; ++p) v += *reinterpret_cast<const floatx4*>(partials + p * size + at);
+  const int64_t m = at / a.N;
+  const int32_t c = (int32_t)(at - m * a.N);
+  if (a.bias != nullptr) v += *reinterpret_cast<const floatx4*>(a.bias + c);
+  if (a.epilogue == kEpiGelu) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = gelu(v[e]);
+  }
+  *reinterpret_cast<floatx4*>(a.y + m * a.y_stride + c) = v;
+}
+
+// Parts K is split into where the output alone gives too few of the 256 CUs a 128 x 64 tile: the
+// most that keep the parts equal, at least four steps long and on a CU each. 1: no split.
+constexpr int kSplitTiles = 160;
+int split_parts(int64_t M, int64_t N, int64_t K) {
+  constexpr int kCus = 256;
+  const int64_t tiles = ((M + 127) / 128) * ((N + 63) / 64), steps = K / kStep;
+  if (tiles >= kSplitTiles || N % 4 != 0) return 1;
+  int parts = 1;
+  for (int p = 2; p * tiles <= kCus && 4 * p <= steps; ++p)
+    if (steps % p == 0) parts = p;
+  return parts;
 }
 
 // Tile shapes and what one tile takes per 32 of K alone on a CU (ns, measured at K = 3072). A CU
@@ -313,8 +353,16 @@ const TileShape& choose_shape(int64_t M, int64_t N) {
 }  // namespace
 }  // namespace tq
 
+extern "C" size_t tq_linear_workspace_size(int32_t M, int32_t N, int32_t K) {
+  using namespace tq;
+  if (M < 1 || N < 1 || K < 1 || K % kStep != 0) return 0;
+  const int parts = split_parts(M, N, K);
+  return parts > 1 ? (size_t)parts * M * N * 4 : 0;
+}
+
 extern "C" tq_status tq_linear(float* y, int64_t y_stride, const float* x, int64_t x_stride, int32_t M, const float* w,
-                               const float* bias, int32_t N, int32_t K, int32_t epilogue, void* stream) {
+                               const float* bias, int32_t N, int32_t K, int32_t epilogue, void* workspace,
+                               size_t workspace_bytes, void* stream) {
   using namespace tq;
   if (M < 0 || N < 1 || K < 1 || epilogue < 0 || epilogue > 1) return TQ_ERR_INVALID_ARGUMENT;
   // 32-bit offsets inside a tile; K in whole steps.
@@ -337,7 +385,26 @@ extern "C" tq_status tq_linear(float* y, int64_t y_stride, const float* x, int64
   a.K = K;
   a.epilogue = epilogue;
   a.vec = N % 4 == 0 && y_stride % 4 == 0 && ((uintptr_t)y | (uintptr_t)bias) % 16 == 0;
+  a.k_part = K;
+  a.parts = 1;
   hipStream_t s = (hipStream_t)stream;
+  const int parts = a.vec ? split_parts(M, N, K) : 1;  // the sum reads and writes whole float4s
+  if (parts > 1) {
+    if (workspace == nullptr || workspace_bytes < tq_linear_workspace_size(M, N, K) || (uintptr_t)workspace % 16 != 0)
+      return TQ_ERR_WORKSPACE;
+    LinearArgs part = a;
+    part.y = static_cast<float*>(workspace);
+    part.y_stride = N;
+    part.bias = nullptr;
+    part.epilogue = kEpiBias;
+    part.k_part = K / parts;
+    part.parts = a.parts = parts;
+    launch<4, 2, 2>(part, s);
+    const int64_t groups = ((int64_t)M * N / 4 + 255) / 256;
+    hipLaunchKernelGGL(linear_sum_kernel, dim3((unsigned)groups), dim3(256), 0, s, a,
+                       static_cast<const float*>(workspace));
+    return check_launch();
+  }
   const TileShape& t = choose_shape(M, N);
   switch (t.wm * 10 + t.nb) {
     case 41: launch<4, 1, 2>(a, s); break;

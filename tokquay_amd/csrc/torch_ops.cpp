@@ -300,9 +300,13 @@ void linear(at::Tensor out, const at::Tensor& x, const at::Tensor& weight, const
               op, ": out must be a float32 [rows, N] tensor on x's device with contiguous rows");
   TORCH_CHECK(M <= 1 || out.stride(0) >= N, op, ": out's rows overlap");
   TORCH_CHECK(M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX, op, ": sizes past int32");
+  // Per call, from torch's allocator: safe on any stream and under graph capture.
+  const size_t bytes = tq_linear_workspace_size((int32_t)M, (int32_t)N, (int32_t)K);
+  at::Tensor workspace;
+  if (bytes > 0) workspace = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
   check(tq_linear(out.data_ptr<float>(), M > 1 ? out.stride(0) : N, x.data_ptr<float>(), M > 1 ? x.stride(0) : K,
                   (int32_t)M, weight.data_ptr<float>(), ptr<float>(bias), (int32_t)N, (int32_t)K, gelu ? 1 : 0,
-                  stream_of(x)),
+                  bytes > 0 ? workspace.data_ptr() : nullptr, bytes, stream_of(x)),
         "tq_linear");
 }
 

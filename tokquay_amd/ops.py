@@ -536,14 +536,23 @@ def uses_nn_layout(rows: int, out_features: int, in_features: int, gelu: bool) -
 # 144 tiles 15.8 -> 18.6; [768, 1600, 1600] 150 tiles 33.8 -> 34.5; [1280, 1024, 1024] 160 tiles 24.9 -> 24.1;
 # [640, 2304, 768] 180 tiles 25.6 -> 19.2; [2048, 768, 768] 192 tiles 26.1 -> 19.9; [2048, 768, 3072] 192 tiles
 # 78.8 -> 66.4; [65, 50257, 768] 786 tiles 69.8 -> 52.7; [8192, 3072, 768] 3,072 tiles 280 -> 191.
+# With fewer tiles, long K is worth splitting over the idle CUs (tq_linear does, and sums the parts in a
+# second launch) from 320 rows on: [384 / 640 / 768 / 1280, 768, 3072] 28.2 / 30.7 / 41.3 / 54.6 -> 21.5 / 27.9 /
+# 33.2 / 46.0, [512, 1024, 4096] 39.8 -> 33.8, [512, 1600, 6400] 105 -> 80. Fewer rows and short K stay with the
+# library: [256 / 300, 768, 3072] 18.9 / 19.4 -> 18.6 / 20.2, [300, 1600, 6400] 59 -> 76, [640, 768, 768]
+# 10.2 -> 15.2.
 ROWS_KERNEL_MIN_TILES = 160
+SPLIT_MAX_TILES, SPLIT_MIN_ROWS, SPLIT_MIN_K = 128, 320, 3072
 _TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
 def uses_rows_kernel(rows: int, out_features: int, in_features: int) -> bool:
     """Whether a linear layer of these sizes runs on ``tq_linear`` (else on the library GEMM)."""
-    return (((rows + 127) >> 7) * ((out_features + 63) >> 6) >= ROWS_KERNEL_MIN_TILES
-            and in_features % 32 == 0 and in_features > 0)  # fmt: skip
+    tiles = ((rows + 127) >> 7) * ((out_features + 63) >> 6)
+    if tiles < ROWS_KERNEL_MIN_TILES and (in_features < SPLIT_MIN_K or rows < SPLIT_MIN_ROWS
+                                          or tiles > SPLIT_MAX_TILES or out_features % 4):  # fmt: skip
+        return False
+    return in_features % 32 == 0 and in_features > 0
 
 
 def _rows_kernel_takes(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None) -> bool:
