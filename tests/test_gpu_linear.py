@@ -114,7 +114,7 @@ def test_rule():
     assert _lib.lib().tq_linear_workspace_size(640, 768, 3072) == 4 * 640 * 768 * 4
     assert not ops.uses_rows_kernel(256, 2304, 768) and not ops.uses_rows_kernel(0, 2304, 768)
     assert ops.uses_rows_kernel(640, 2304, 768) and ops.uses_rows_kernel(2048, 768, 3072)
-    assert ops.uses_rows_kernel(65, 50257, 768)
+    assert ops.uses_rows_kernel(65, 50257, 768) and not ops.uses_rows_kernel(63, 50257, 768)
     assert not ops.uses_rows_kernel(8192, 3072, 776) and not ops.uses_rows_kernel(8192, 3072, 0)
 
 

@@ -541,7 +541,10 @@ def uses_nn_layout(rows: int, out_features: int, in_features: int, gelu: bool) -
 # 33.2 / 46.0, [512, 1024, 4096] 39.8 -> 33.8, [512, 1600, 6400] 105 -> 80. Fewer rows and short K stay with the
 # library: [256 / 300, 768, 3072] 18.9 / 19.4 -> 18.6 / 20.2, [300, 1600, 6400] 59 -> 76, [640, 768, 768]
 # 10.2 -> 15.2.
+# Fewer than 64 rows leave the 128-row tiles mostly padding, however many they are: the LM head [rows, 50257,
+# 768] 8 / 32 / 48 / 64 / 128 rows 33 / 37 / 45 / 67 / 104 -> 53 / 52 / 55 / 57 / 70.
 ROWS_KERNEL_MIN_TILES = 160
+ROWS_KERNEL_MIN_ROWS = 64
 SPLIT_MAX_TILES, SPLIT_MIN_ROWS, SPLIT_MIN_K = 128, 320, 3072
 _TENSORS = (torch.Tensor, torch.nn.Parameter)
 
@@ -549,6 +552,8 @@ _TENSORS = (torch.Tensor, torch.nn.Parameter)
 def uses_rows_kernel(rows: int, out_features: int, in_features: int) -> bool:
     """Whether a linear layer of these sizes runs on ``tq_linear`` (else on the library GEMM)."""
     tiles = ((rows + 127) >> 7) * ((out_features + 63) >> 6)
+    if rows < ROWS_KERNEL_MIN_ROWS:
+        return False
     if tiles < ROWS_KERNEL_MIN_TILES and (in_features < SPLIT_MIN_K or rows < SPLIT_MIN_ROWS
                                           or tiles > SPLIT_MAX_TILES or out_features % 4):  # fmt: skip
         return False
