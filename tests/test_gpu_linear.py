@@ -139,3 +139,52 @@ def test_calls_the_kernel_does_not_take_run_as_before(monkeypatch):
         assert not taken
         ops.linear(x, lin)
         assert len(taken) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 7, 16, 17, 100, 320, 321])
+def test_eager_few_rows_and_the_head(rows, monkeypatch):
+    """Few rows: the wide layers run on tq_linear outside a capture and on the library inside one; the
+    LM head on the library below 64 rows. All within fp32's bound."""
+    x, w, b = _inputs(rows, 3072, 768)
+    lin = torch.nn.Linear(768, 3072).cuda().requires_grad_(False)
+    lin.weight.copy_(w), lin.bias.copy_(b)
+    _check(ops.linear(x, lin), x, w, b)
+    _check(ops.linear(x, lin, gelu=True), x, w, b, gelu=True)
+    assert ops._rows_kernel_takes(x, lin.weight, lin.bias) == (rows <= 320)
+    taken = []
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: taken.append(1) or True)
+    assert not ops._rows_kernel_takes(x, lin.weight, lin.bias) and len(taken) == (rows <= 320)
+    monkeypatch.undo()
+    square = torch.nn.Linear(768, 768).cuda().requires_grad_(False)
+    assert ops._rows_kernel_takes(x, square.weight, square.bias) == (rows <= 128)
+    _check(ops.linear(x, square), x, square.weight, square.bias)
+    assert not ops._saves_host_time(rows, 32000, 768)  # an LM head's weights are the GPU's time
+    wide = (torch.randn(50257, 768, generator=torch.Generator().manual_seed(rows)) * 0.02).cuda()
+    assert ops._rows_kernel_takes(x, wide, None) == (rows >= 64)
+    _check(ops.lm_head(x, wide), x, wide, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [100, 256])
+@pytest.mark.parametrize("prepared", ["eager", "captured form"])
+def test_one_run_prepares_a_capture(rows, prepared):
+    """The layers of a decode step captured after one run, eager or in the captured form: every replay
+    gives the library's result (256 rows: through the transposed weights) on what the inputs hold."""
+    up, down = torch.nn.Linear(768, 3072).cuda(), torch.nn.Linear(3072, 768).cuda()
+    x = torch.randn(rows, 768, device="cuda")
+    f = lambda: ops.linear(ops.linear(x, up, gelu=True), down)  # noqa: E731
+    with torch.no_grad():
+        if prepared == "eager":
+            f()
+        else:
+            with ops.captured_form():
+                f()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = f()
+        for _ in range(3):
+            x.normal_()
+            graph.replay()
+            torch.testing.assert_close(y, f(), rtol=1e-4, atol=1e-4)
+            torch.cuda.synchronize()

@@ -8,7 +8,7 @@ bucket (powers of two) into a HIP graph and replays it. Buckets of at most 64
 rows run the fused small-batch path (``GPT2.skinny_logits``: each linear of a
 block with its LayerNorm / GELU / residual add in one ``tq_skinny_linear`` launch,
 about 65 launches per step; the LM head fused with ``ln_f`` up to 16 rows, else
-``ln_f`` alone and the head on hipBLASLt); larger buckets the library GEMMs with
+``ln_f`` alone and the head through ``ops.lm_head``); larger buckets ``ops.linear`` with
 ``tq_add_layernorm``. A step whose rows are all greedy at most 16 rows replays an
 ids-only graph instead: the LM head with ``ln_f`` and the argmax in one
 ``tq_skinny_linear_argmax`` launch, no logits written.
@@ -177,7 +177,8 @@ class DecodeGraphs:
         tokens = s.tokens.clone()  # the warm-up runs overwrite what this step's source rows read
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side):  # warm-up launches (same inputs: the K/V writes are idempotent)
+        # Warm-up launches of what is captured (same inputs: the K/V writes are idempotent).
+        with torch.cuda.stream(side), ops.captured_form():
             for _ in range(2):
                 self._forward(rows, ids_only)
                 s.tokens.copy_(tokens)

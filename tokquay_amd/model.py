@@ -57,7 +57,7 @@ class MLP(nn.Module):
         self.c_proj = nn.Linear(4 * cfg.n_embd, cfg.n_embd)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        # GELU (tanh form, tokquay/model.py:107) as the GEMM's epilogue on the GPU (hipBLASLt): one launch
+        # GELU (tanh form, tokquay/model.py:107) as the product's epilogue on the GPU: one launch
         # instead of two. On the CPU torch's fused path computes the erf form, so ops.linear applies it apart.
         return ops.linear(ops.linear(x, self.c_fc, gelu=True), self.c_proj)
 
@@ -133,8 +133,8 @@ class GPT2(nn.Module):
     def skinny_logits(self, x: torch.Tensor, cache) -> torch.Tensor:
         """Logits ``[M, vocab]`` of ``M <= ops.SKINNY_MAX_ROWS`` rows from their embeddings ``x``
         (:meth:`skinny_trunk`), then the tied LM head with ``ln_f`` in front (tokquay/model.py:180-181),
-        fused up to ``ops.SKINNY_LM_HEAD_MAX_ROWS`` rows, else ``ln_f`` on its own and the head on
-        hipBLASLt."""
+        fused up to ``ops.SKINNY_LM_HEAD_MAX_ROWS`` rows, else ``ln_f`` on its own and the head
+        through ``ops.lm_head``."""
         x = self.skinny_trunk(x, cache)
         if x.shape[0] <= ops.SKINNY_LM_HEAD_MAX_ROWS:
             return ops.skinny_linear(x, self.wte.weight, None, ln=(self.ln_f.weight, self.ln_f.bias, self.ln_f.eps))

@@ -16,7 +16,9 @@ Shapes (fp32 unless noted; ``H`` heads of ``D = 64`` dims):
 
 from __future__ import annotations
 
+import contextlib
 import math
+import threading
 
 import torch
 
@@ -546,7 +548,29 @@ def uses_nn_layout(rows: int, out_features: int, in_features: int, gelu: bool) -
 ROWS_KERNEL_MIN_TILES = 160
 ROWS_KERNEL_MIN_ROWS = 64
 SPLIT_MAX_TILES, SPLIT_MIN_ROWS, SPLIT_MIN_K = 128, 320, 3072
+# Up to some rows an eager step is bound by the host: the library call takes it about 21 us, tq_linear
+# about 9, for about the same GPU time in the wide layers ([64-256, 3072, 768] 10-19 -> 12-19 us,
+# [64-256, 768, 3072] 11-19 -> 13-19): the MLP over 256 rows 44 -> 34 us a call, over 64 45 -> 27. The
+# narrower ones ([2304, 768] 10-14 -> 11-14 us, [768, 768] 7 -> 10 at 64-128 rows) follow up to 128 rows; at
+# 256 (14.5 -> 16, 7 -> 12) the layer with its attention is bound by the GPU: 182.0 -> 182.9 us.
+# Captured steps, whose launches cost the host nothing, stay with the library.
+EAGER_ROWS, EAGER_WIDTH = 320, 3072
+EAGER_NARROW_ROWS, EAGER_NARROW_WIDTH = 128, 768
+EAGER_MAX_WEIGHTS = 1600 * 6400  # [16-128, 1600, 6400] 20-38 -> 22-27 us; the LM head (above) is bound by the GPU
 _TENSORS = (torch.Tensor, torch.nn.Parameter)
+_captured = threading.local()
+
+
+@contextlib.contextmanager
+def captured_form():
+    """The calling thread's calls inside run what they would run under capture: for the runs that
+    prepare one (library kernels loaded, weight copies made)."""
+    before = getattr(_captured, "form", False)
+    _captured.form = True
+    try:
+        yield
+    finally:
+        _captured.form = before
 
 
 def uses_rows_kernel(rows: int, out_features: int, in_features: int) -> bool:
@@ -560,14 +584,23 @@ def uses_rows_kernel(rows: int, out_features: int, in_features: int) -> bool:
     return in_features % 32 == 0 and in_features > 0
 
 
+def _saves_host_time(rows: int, out_features: int, in_features: int) -> bool:
+    """Whether an eager linear layer of few rows runs on ``tq_linear`` for its cheaper call."""
+    return (0 < rows <= EAGER_ROWS
+            and max(out_features, in_features) >= (EAGER_WIDTH if rows > EAGER_NARROW_ROWS else EAGER_NARROW_WIDTH)
+            and out_features * in_features <= EAGER_MAX_WEIGHTS and in_features % 32 == 0 and out_features % 4 == 0
+            and not getattr(_captured, "form", False) and not torch.cuda.is_current_stream_capturing())  # fmt: skip
+
+
 def _rows_kernel_takes(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None) -> bool:
-    """Whether ``x @ w.T + bias`` may go to ``tq_linear``: enough tiles (``uses_rows_kernel``), plain
-    float32 tensors on one HIP device in the layout it reads, and nothing that must see torch's own
-    product (a gradient, a functorch transform, forward-mode AD, a tensor subclass)."""
+    """Whether ``x @ w.T + bias`` goes to ``tq_linear``: by its sizes (``uses_rows_kernel``,
+    ``_saves_host_time``), for plain float32 tensors on one HIP device in the layout it reads, and if
+    nothing must see torch's own product (a gradient, a functorch transform, forward-mode AD, a tensor
+    subclass)."""
     n, k = w.shape
-    if not uses_rows_kernel(x.size(0), n, k):  # most small calls end here: the cheapest test first
-        return False
     if x.dim() != 2 or x.size(1) != k:
+        return False
+    if not uses_rows_kernel(x.size(0), n, k) and not _saves_host_time(x.size(0), n, k):
         return False
     ts = (x, w) if bias is None else (x, w, bias)
     if any(type(t) not in _TENSORS or t.dtype != torch.float32 or t.device != x.device for t in ts):
@@ -604,8 +637,10 @@ def linear(x: torch.Tensor, layer: torch.nn.Linear, gelu: bool = False) -> torch
     if not x.is_cuda:
         y = torch.nn.functional.linear(x, weight, bias)
         return torch.nn.functional.gelu(y, approximate="tanh") if gelu else y
-    if _rows_kernel_takes(x, weight, bias):
-        return _rows_linear(x, weight, bias, gelu)
     out_f, in_f = weight.shape
     nn_layout = uses_nn_layout(x.shape[0], out_f, in_f, gelu)
+    if _rows_kernel_takes(x, weight, bias):
+        if nn_layout:
+            transposed_weight(layer)  # a capture of this shape needs it, and one eager run is to prepare that
+        return _rows_linear(x, weight, bias, gelu)
     return _gemm(x, transposed_weight(layer) if nn_layout else weight.t(), bias, gelu)
