@@ -27,7 +27,7 @@
 // log2 e, so p = 2^(s - m) on v_exp_f32). The max is lazy: it moves, and the
 // accumulators are rescaled, only when a score passes it by more than 2^8.
 //
-// With block size 16 or 32 the key loop is software-pipelined: each wave issues the
+// With block size 8, 16 or 32 the key loop is software-pipelined: each wave issues the
 // next key tile's K/V loads (buffer loads off descriptors on the block's K and V
 // tiles) before the current tile's math. The MFMA results stay in VGPRs (built
 // with -amdgpu-mfma-vgpr-form), so the per-tile rescale and the softmax read them
@@ -121,7 +121,8 @@ __device__ __forceinline__ float max_over_lane_groups(float v) {
 // the direct loads: there the registers place_k() takes cost a wave per SIMD. Measured us (direct ->
 // place_k()): 4 chunks of 256 rows at 0 / 256 / 512 10.5 / 18.7 / 27.0 -> 10.2 / 18.2 / 25.5, 8 x 256 behind
 // 700 keys 64.7 -> 58.2, a mixed launch of 4 x 250-256 rows at 512 beside 128 decode rows 71.6 -> 64.6;
-// one wave per tile: 7 prompts of 33-511 rows 26.7 -> 28.0, two tiles per wave 44.0 -> 50.0.
+// one wave per tile: 7 prompts of 33-511 rows 26.7 -> 28.0, two tiles per wave 44.0 -> 50.0. (Launches whose
+// whole context is a few tiles pay for the trip through LDS: a prompt of 30 rows 4.5 -> 4.6.)
 template <int BS, bool ROWS>
 __device__ __forceinline__ void load_kv_block_tile(const PrefillArgs& a, const float* head_base, int32_t blk,
                                                    int kt, int kend, int j, int g, float (&kreg)[16],
@@ -149,18 +150,61 @@ __device__ __forceinline__ void load_kv_block_tile(const PrefillArgs& a, const f
   }
 }
 
+// Block size 8: a 16-key tile is two blocks, blk0 and blk1, each with its own two descriptors. Every load
+// covers four whole rows of one block, K's as with ROWS and V's too: load s gives lane (j, g) V row 4 s + g,
+// so the tile's keys enter the products in the order of pair_row() instead of their own. The general loop
+// (an address and a table entry per lane and row, nothing in flight ahead) was bound by its address
+// arithmetic and load latency. Measured us (general -> pairs): 4 chunks of 256 rows at 0 / 256 / 512
+// 14.9 / 29.0 / 43.1 -> 10.2 / 17.7 / 25.8, 8 x 256 behind 700 keys 110 -> 59, a prompt of 64 rows 6.0 -> 4.9,
+// 250 prompts of 60-64 rows 54 -> 48; 4 x 250-256 rows at 0 / 512 beside 128 decode rows 77 / 97 -> 77 / 82.
+// All launches place K through LDS here: with the direct loads a lane's row would need its own descriptor.
+__device__ __forceinline__ void load_kv_block_pair(const PrefillArgs& a, const float* head_base, int32_t blk0,
+                                                   int32_t blk1, int kt, int kend, int j, int g, float (&kreg)[16],
+                                                   float4 (&vreg)[4]) {
+  constexpr int kRowBytes = kHeadDim * 4;
+  const uint32_t off = (uint32_t)(g * kHeadDim + 4 * j) * 4u;
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    const int32_t blk = half == 0 ? blk0 : blk1;
+    int rows = blk < 0 || kt + 8 * half >= kend ? 0 : min(8, kend - kt - 8 * half);
+    rows = __builtin_amdgcn_readfirstlane(rows);
+    const float* kb = head_base + (int64_t)(blk < 0 ? 0 : blk) * a.block_stride;
+    const __amdgpu_buffer_rsrc_t kd =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kb), (short)0, rows * kRowBytes, kBufferWord3);
+    const __amdgpu_buffer_rsrc_t vd = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kb + a.kv_stride),
+                                                                        (short)0, rows * kRowBytes, kBufferWord3);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const auto x = __builtin_amdgcn_raw_buffer_load_b128(kd, off + (uint32_t)(4 * t * kRowBytes), 0, 0);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) kreg[4 * (2 * half + t) + c] = __uint_as_float(x[c]);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const auto x = __builtin_amdgcn_raw_buffer_load_b128(vd, off + (uint32_t)(4 * t * kRowBytes), 0, 0);
+      vreg[2 * half + t] =
+          make_float4(__uint_as_float(x[0]), __uint_as_float(x[1]), __uint_as_float(x[2]), __uint_as_float(x[3]));
+    }
+  }
+}
+
+// The tile row at place 4 g + s of the products of a block pair: V's loads put row 4 s + g there.
+__device__ __forceinline__ constexpr int pair_row(int place) { return 4 * (place & 3) + (place >> 2); }
+
 // Moves a K tile loaded with ROWS to the QK product's A operand, through the wave's own
-// 4 KiB of LDS: kout[s] of lane (j, g) = K[row j][16 g + s]. Float4 c of row r sits in slot 16 r + (c ^ r):
-// neither side has bank conflicts.
+// 4 KiB of LDS: kout[s] of lane (j, g) = K[row][16 g + s] of the row at place j. Float4 c of row r sits in slot
+// 16 r + (c ^ r): neither side has bank conflicts.
+template <bool PAIR>
 __device__ __forceinline__ void place_k(float4* slots, int j, int g, const float (&kreg)[16], float (&kout)[16]) {
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int r = 4 * t + g;
     slots[16 * r + (j ^ r)] = make_float4(kreg[4 * t], kreg[4 * t + 1], kreg[4 * t + 2], kreg[4 * t + 3]);
   }
+  const int row = PAIR ? pair_row(j) : j;
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
-    const float4 x = slots[16 * j + ((4 * g + v) ^ j)];
+    const float4 x = slots[16 * row + ((4 * g + v) ^ row)];
     kout[4 * v + 0] = x.x;
     kout[4 * v + 1] = x.y;
     kout[4 * v + 2] = x.z;
@@ -171,14 +215,14 @@ __device__ __forceinline__ void place_k(float4* slots, int j, int g, const float
 // The work of prefill workgroup `dispatch` (its KS waves): QH consecutive query tiles of one head
 // of one sequence, or nothing for a padding workgroup. QH = 2 (one wave per workgroup only) feeds
 // each key tile's loads to twice the MFMAs and gives the wave two independent softmax chains.
-// PIPE: the software-pipelined key loop (block sizes 16 and 32). The mixed launch keeps the plain
+// PIPE: the software-pipelined key loop (block sizes 8, 16 and 32). The mixed launch keeps the plain
 // loop: with the pipelined one (126 VGPRs, its decode workgroups still at 4 waves per SIMD) the
 // steps of four 256-token prompt chunks beside 128 decoding sequences ran from 3 % faster to 2 %
 // slower depending on the chunk.
 template <int BS_CT, int KS, int QH = 1, bool PIPE = (BS_CT > 0)>
 __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int dispatch) {
-  static_assert(BS_CT == 0 || BS_CT % kTile == 0, "a key tile lies in one block");
-  static_assert(!PIPE || BS_CT > 0, "the pipelined key loop reads one block per key tile");
+  static_assert(BS_CT == 0 || BS_CT == 8 || BS_CT % kTile == 0, "a key tile lies in one block, or is two");
+  static_assert(!PIPE || BS_CT > 0, "the pipelined key loop reads whole blocks");
   static_assert(QH == 1 || KS == 1, "two query tiles per wave only without a key split");
   const int lane = threadIdx.x & (kWave - 1);
   // Wave-uniform by construction; readfirstlane lets the compiler keep the key-tile loop
@@ -294,12 +338,13 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
   // running-maximum test on each lane's own four scores (the lane-group maximum only when some
   // lane's test fires), max as v_maximum3_f32 (no operand canonicalization), and one ballot
   // for all of the wave's query tiles.
-  constexpr bool kPlaceK = BS_CT > 0 && (KS > 1 || !PIPE);
+  constexpr bool kPair = BS_CT == 8;
+  constexpr bool kPlaceK = BS_CT > 0 && (KS > 1 || !PIPE || kPair);
   __shared__ float4 s_k[KS][kPlaceK ? kTile * kHeadDim / 4 : 1];
   auto consume = [&](int kt, const float (&kload)[16], const float4 (&vreg)[4]) {
       float kreg[16];
       if constexpr (kPlaceK) {
-        place_k(s_k[wave], j, g, kload, kreg);
+        place_k<kPair>(s_k[wave], j, g, kload, kreg);
       } else {
   #pragma unroll
         for (int s = 0; s < 16; ++s) kreg[s] = kload[s];
@@ -312,14 +357,15 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
   #pragma unroll
         for (int u = 0; u < QH; ++u) st[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kreg[s], qreg[u][s], st[u], 0, 0, 0);
       }
-      // sm[u][r] = S^T[key kt + 4g + r][query j] in log2 units, -inf past the diagonal.
+      // sm[u][r] = S^T[key kt + 4g + r (a block pair's: kt + 4r + g)][query j] in log2 units, -inf past the
+      // diagonal.
       float sm[QH][4], lmax[QH];
       bool grow_any = false;
   #pragma unroll
       for (int u = 0; u < QH; ++u) {
         if (kt + kTile - 1 > qpos_lo[u]) {  // uniform: the key tile crosses this query tile's diagonal
   #pragma unroll
-          for (int r = 0; r < 4; ++r) sm[u][r] = kt + 4 * g + r <= qpos[u] ? st[u][r] : -INFINITY;
+          for (int r = 0; r < 4; ++r) sm[u][r] = kt + (kPair ? 4 * r + g : 4 * g + r) <= qpos[u] ? st[u][r] : -INFINITY;
         } else {
   #pragma unroll
           for (int r = 0; r < 4; ++r) sm[u][r] = st[u][r];
@@ -365,6 +411,17 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
       }
   };
 
+  // A key tile's loads, `at` the table entry's lane of tb_id (a pair's second block is in the next lane:
+  // tiles start at even entries).
+  auto load_tile = [&](int32_t tb_id, int at, int kt, float(&kreg)[16], float4(&vreg)[4]) {
+    if constexpr (kPair)
+      load_kv_block_pair(a, head_base, __builtin_amdgcn_readlane(tb_id, at), __builtin_amdgcn_readlane(tb_id, at + 1),
+                         kt, kend, j, g, kreg, vreg);
+    else if constexpr (BS_CT > 0)
+      load_kv_block_tile<BS_CT, kPlaceK>(a, head_base, __builtin_amdgcn_readlane(tb_id, at), kt, kend, j, g, kreg,
+                                         vreg);
+  };
+
   if constexpr (PIPE) {
     // The ids of 64 consecutive blocks are held one per lane and fetched per tile with
     // v_readlane (no table loads in the loop); the lane copy is refreshed when the
@@ -385,7 +442,7 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
           else flag_error(a.d_error, TQ_DEVERR_BLOCK_ID);
         }
       }
-      load_kv_block_tile<BS_CT, kPlaceK>(a, head_base, __builtin_amdgcn_readlane(tb_id, ti - tb_base), kt, kend, j, g, kreg, vreg);
+      load_tile(tb_id, ti - tb_base, kt, kreg, vreg);
     };
     const int step = KS * kTile;
     int kt = wave * kTile;
@@ -447,7 +504,7 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
             else flag_error(a.d_error, TQ_DEVERR_BLOCK_ID);
           }
         }
-        load_kv_block_tile<BS_CT, kPlaceK>(a, head_base, __builtin_amdgcn_readlane(tb_id, ti - tb_base), kt, kend, j, g, kreg, vreg);
+        load_tile(tb_id, ti - tb_base, kt, kreg, vreg);
       } else {
         load_kv_tile<BS_CT>(a, bt, head_base, bs, kt, kend, j, g, kreg, vreg);
       }
@@ -802,6 +859,7 @@ extern "C" tq_status tq_paged_prefill(float* out, int64_t out_row_stride, const 
     return check_launch();
   }
   switch (block_size) {
+    case 8: launch_prefill<8>(a, s, timing.start, timing.stop); break;
     case 16: launch_prefill<16>(a, s, timing.start, timing.stop); break;
     case 32: launch_prefill<32>(a, s, timing.start, timing.stop); break;
     default: launch_prefill<0>(a, s, timing.start, timing.stop); break;
@@ -902,6 +960,7 @@ extern "C" tq_status tq_paged_mixed(float* dec_out, int64_t dec_out_row_stride, 
   const int32_t g32 = (int32_t)groups, u32 = (int32_t)units;
   hipEvent_t stop = merge ? nullptr : timing.stop;
   switch (block_size) {
+    case 8: launch_mixed<0, 8>(pa, da, ks, g32, u32, s, timing.start, stop); break;
     case 16: launch_mixed<16, 16>(pa, da, ks, g32, u32, s, timing.start, stop); break;
     case 32: launch_mixed<32, 32>(pa, da, ks, g32, u32, s, timing.start, stop); break;
     default: launch_mixed<0, 0>(pa, da, ks, g32, u32, s, timing.start, stop); break;
