@@ -355,7 +355,7 @@ def prefill_batch(seed: int = 32, reps: int = 3) -> dict:
     us = statistics.median(times)
     return {"workload": f"one prefill step: 32 prompts U[256,1024] at start 0 ({sum(lens)} rows), block 16, "
                         "12 layers; median launch over the layers of 3 runs",
-            "kernel": "tq_paged_prefill (fp32 MFMA 16x16x4; one wave per workgroup, two query tiles per wave)",
+            "kernel": "tq_paged_prefill (128-query workgroups, fp32 products as six bf16 MFMA 32x32x16)",
             "bound": "mfma", "us_per_launch": round(us, 2), "mflop_per_launch": round(flops / 1e6, 1),
             "achieved": round(flops / us / 1e6, 2), "peak": MFMA_FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": round(flops / us / 1e6 / MFMA_FP32_PEAK_TFLOPS, 4)}  # fmt: skip

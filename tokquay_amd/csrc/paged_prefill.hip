@@ -120,9 +120,10 @@ __device__ __forceinline__ float max_over_lane_groups(float v) {
 // place_k() gets the rows into place through LDS. The launches with one pipelined wave per tile keep
 // the direct loads: there the registers place_k() takes cost a wave per SIMD. Measured us (direct ->
 // place_k()): 4 chunks of 256 rows at 0 / 256 / 512 10.5 / 18.7 / 27.0 -> 10.2 / 18.2 / 25.5, 8 x 256 behind
-// 700 keys 64.7 -> 58.2, a mixed launch of 4 x 250-256 rows at 512 beside 128 decode rows 71.6 -> 64.6;
-// one wave per tile: 7 prompts of 33-511 rows 26.7 -> 28.0, two tiles per wave 44.0 -> 50.0. (Launches whose
-// whole context is a few tiles pay for the trip through LDS: a prompt of 30 rows 4.5 -> 4.6.)
+// 700 keys 64.7 -> 58.2, a mixed launch of 4 x 250-256 rows at 512 beside 128 decode rows 71.6 -> 64.6 (at 0 / 256 /
+// 384 / 700 57.8 / 60.6 / 63.8 / 81.5 -> 58.7 / 61.2 / 61.7 / 76.0); one wave per tile: 7 prompts of 33-511 rows
+// 26.7 -> 28.0, two tiles per wave 44.0 -> 50.0. Short contexts pay a little for the trip through LDS (a prompt of
+// 30 rows 4.5 -> 4.6).
 template <int BS, bool ROWS>
 __device__ __forceinline__ void load_kv_block_tile(const PrefillArgs& a, const float* head_base, int32_t blk,
                                                    int kt, int kend, int j, int g, float (&kreg)[16],
