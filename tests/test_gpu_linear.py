@@ -188,3 +188,16 @@ def test_one_run_prepares_a_capture(rows, prepared):
             graph.replay()
             torch.testing.assert_close(y, f(), rtol=1e-4, atol=1e-4)
             torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs two GPUs")
+def test_runs_on_its_tensors_device():
+    """With another device current, the launch goes to the tensors' device and its stream."""
+    x, w, b = _inputs(640, 2304, 768)
+    want = ops._rows_linear(x, w, b, False)
+    x, w, b = (t.to("cuda:1") for t in (x, w, b))
+    with torch.cuda.device(0):
+        x.mul_(2.0).mul_(0.5)  # queued on cuda:1's stream in front of the product
+        assert torch.equal(ops._rows_linear(x, w, b, False).cpu(), want.cpu())
+        assert torch.cuda.current_device() == 0

@@ -11,6 +11,7 @@
 // variants, the pool) in place, annotated as mutations.
 
 #include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
 
@@ -29,7 +30,18 @@ void check(tq_status s, const char* what) {
   TORCH_CHECK(false, msg);
 }
 
-void* stream_of(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+// The current stream of t's device, which is the current device until the end of the expression that names it:
+// the handle of a device's default stream is null, and a launch on null goes to whichever device is current.
+class stream_of {
+ public:
+  explicit stream_of(const at::Tensor& t)
+      : guard_(t.device()), stream_(c10::hip::getCurrentHIPStream(t.device().index()).stream()) {}
+  operator void*() const { return stream_; }
+
+ private:
+  c10::DeviceGuard guard_;
+  void* stream_;
+};
 
 // ---- argument checks: everything a kernel would read or write past is refused before any launch.
 // Values inside the tensors (block ids, slots, lengths, orders) are checked by the kernels
