@@ -358,7 +358,8 @@ tq_status tq_linear(float* y, int64_t y_stride, const float* x, int64_t x_stride
 
 /* Bytes of workspace tq_linear needs for these sizes (0 for most: only outputs of too few tiles
  * to fill the GPU are computed in parts of K). 16-byte aligned; its contents need not start at
- * zero. A call whose y or bias is not 16-byte aligned uses none. */
+ * zero. A call whose y or y_stride is not 16-byte aligned uses none, and one whose bias is not can do
+ * without (workspace null). */
 size_t tq_linear_workspace_size(int32_t M, int32_t N, int32_t K);
 
 /*

@@ -104,8 +104,20 @@ def test_parts_of_k_follow_fp32_and_need_their_workspace():
     assert L.tq_linear(*args, y.data_ptr(), 8 * 130 * 512 * 4 - 1, 0) == 3
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("gelu", [False, True])
+def test_parts_of_k_take_any_bias(gelu):
+    """A bias off a 16-byte boundary does not keep K from being split: same bits."""
+    x, w, b = _inputs(130, 512, 1024)
+    want = ops._rows_linear(x, w, b, gelu)
+    for off in (1, 2, 3):
+        flat = torch.zeros(520, device="cuda")
+        flat[off : off + 512] = b
+        assert torch.equal(ops._rows_linear(x, w, flat[off : off + 512], gelu), want)
+
+
 def test_rule():
-    """Few tiles, K not in whole steps: the library; many, or long K to split: tq_linear."""
+    """Few tiles, K not in whole steps: the library; many, or long K to split over the CUs: tq_linear."""
     assert ops.uses_rows_kernel(320, 768, 3072) and not ops.uses_rows_kernel(319, 768, 3072)
     assert not ops.uses_rows_kernel(640, 768, 768) and not ops.uses_rows_kernel(640, 766, 3072)
     assert not ops.uses_rows_kernel(1536, 768, 3072)  # 144 tiles: neither enough nor few enough for two parts
@@ -114,6 +126,10 @@ def test_rule():
     assert _lib.lib().tq_linear_workspace_size(640, 768, 3072) == 4 * 640 * 768 * 4
     assert not ops.uses_rows_kernel(256, 2304, 768) and not ops.uses_rows_kernel(0, 2304, 768)
     assert ops.uses_rows_kernel(640, 2304, 768) and ops.uses_rows_kernel(2048, 768, 3072)
+    # K that cannot be split (97, 103 steps of 32), or into too few parts for the CUs: the library.
+    for m, n, k in ((320, 768, 3104), (320, 768, 3296), (640, 768, 3136), (320, 1600, 6400), (320, 768, 8192)):
+        assert not ops.uses_rows_kernel(m, n, k)
+    assert ops.uses_rows_kernel(512, 1600, 6400) and ops.uses_rows_kernel(320, 768, 3136)
     assert ops.uses_rows_kernel(65, 50257, 768) and not ops.uses_rows_kernel(63, 50257, 768)
     assert not ops.uses_rows_kernel(8192, 3072, 776) and not ops.uses_rows_kernel(8192, 3072, 0)
 

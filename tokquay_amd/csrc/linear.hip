@@ -307,7 +307,10 @@ __global__ __launch_bounds__(256) void linear_sum_kernel(const LinearArgs a, con
   for (int p = 1; p < a.parts; ++p) v += *reinterpret_cast<const floatx4*>(partials + p * size + at);
   const int64_t m = at / a.N;
   const int32_t c = (int32_t)(at - m * a.N);
-  if (a.bias != nullptr) v += *reinterpret_cast<const floatx4*>(a.bias + c);
+  if (a.bias != nullptr) {  // any alignment
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += a.bias[c + e];
+  }
   if (a.epilogue == kEpiGelu) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = gelu(v[e]);
@@ -384,11 +387,13 @@ extern "C" tq_status tq_linear(float* y, int64_t y_stride, const float* x, int64
   a.N = N;
   a.K = K;
   a.epilogue = epilogue;
-  a.vec = N % 4 == 0 && y_stride % 4 == 0 && ((uintptr_t)y | (uintptr_t)bias) % 16 == 0;
+  const bool vec_y = N % 4 == 0 && y_stride % 4 == 0 && (uintptr_t)y % 16 == 0;
+  a.vec = vec_y && (uintptr_t)bias % 16 == 0;
   a.k_part = K;
   a.parts = 1;
   hipStream_t s = (hipStream_t)stream;
-  const int parts = a.vec ? split_parts(M, N, K) : 1;  // the sum reads and writes whole float4s
+  // The sum writes whole float4s; an unaligned bias alone does not need the split's workspace.
+  const int parts = vec_y && (a.vec || workspace != nullptr) ? split_parts(M, N, K) : 1;
   if (parts > 1) {
     if (workspace == nullptr || workspace_bytes < tq_linear_workspace_size(M, N, K) || (uintptr_t)workspace % 16 != 0)
       return TQ_ERR_WORKSPACE;
@@ -396,6 +401,7 @@ extern "C" tq_status tq_linear(float* y, int64_t y_stride, const float* x, int64
     part.y = static_cast<float*>(workspace);
     part.y_stride = N;
     part.bias = nullptr;
+    part.vec = 1;
     part.epilogue = kEpiBias;
     part.k_part = K / parts;
     part.parts = a.parts = parts;

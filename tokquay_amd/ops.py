@@ -17,6 +17,7 @@ Shapes (fp32 unless noted; ``H`` heads of ``D = 64`` dims):
 from __future__ import annotations
 
 import contextlib
+import functools
 import math
 import threading
 
@@ -539,15 +540,16 @@ def uses_nn_layout(rows: int, out_features: int, in_features: int, gelu: bool) -
 # [640, 2304, 768] 180 tiles 25.6 -> 19.2; [2048, 768, 768] 192 tiles 26.1 -> 19.9; [2048, 768, 3072] 192 tiles
 # 78.8 -> 66.4; [65, 50257, 768] 786 tiles 69.8 -> 52.7; [8192, 3072, 768] 3,072 tiles 280 -> 191.
 # With fewer tiles, long K is worth splitting over the idle CUs (tq_linear does, and sums the parts in a
-# second launch) from 320 rows on: [384 / 640 / 768 / 1280, 768, 3072] 28.2 / 30.7 / 41.3 / 54.6 -> 21.5 / 27.9 /
-# 33.2 / 46.0, [512, 1024, 4096] 39.8 -> 33.8, [512, 1600, 6400] 105 -> 80. Fewer rows and short K stay with the
-# library: [256 / 300, 768, 3072] 18.9 / 19.4 -> 18.6 / 20.2, [300, 1600, 6400] 59 -> 76, [640, 768, 768]
-# 10.2 -> 15.2.
+# second launch) from 320 rows on, where the parts give as many CUs work as that: [384 / 640 / 768 / 1280, 768,
+# 3072] 28.2 / 30.7 / 41.3 / 54.6 -> 21.5 / 27.9 / 33.2 / 46.0, [512, 1024, 4096] 37.7 -> 33.5, [512, 1600, 6400] 96 -> 73,
+# but [320, 1600, 6400] (150 parts in all) 54 -> 70, [640, 768, 3136] (120) 31 -> 37 and [320, 768, 3104] (K of 97
+# steps: no split) 28 -> 56. Fewer rows and short K stay with the library: [256 / 300, 768, 3072] 18.9 / 19.4 -> 18.6 /
+# 20.2, [300, 1600, 6400] 59 -> 76, [640, 768, 768] 10.2 -> 15.2.
 # Fewer than 64 rows leave the 128-row tiles mostly padding, however many they are: the LM head [rows, 50257,
 # 768] 8 / 32 / 48 / 64 / 128 rows 33 / 37 / 45 / 67 / 104 -> 53 / 52 / 55 / 57 / 70.
 ROWS_KERNEL_MIN_TILES = 160
 ROWS_KERNEL_MIN_ROWS = 64
-SPLIT_MAX_TILES, SPLIT_MIN_ROWS, SPLIT_MIN_K = 128, 320, 3072
+SPLIT_MIN_ROWS, SPLIT_MIN_K = 320, 3072
 # Up to some rows an eager step is bound by the host: the library call takes it about 21 us, tq_linear
 # about 9, for about the same GPU time in the wide layers ([64-256, 3072, 768] 10-19 -> 12-19 us,
 # [64-256, 768, 3072] 11-19 -> 13-19): the MLP over 256 rows 44 -> 34 us a call, over 64 45 -> 27. The
@@ -573,15 +575,23 @@ def captured_form():
         _captured.form = before
 
 
+@functools.lru_cache(maxsize=1024)
+def _split_parts(rows: int, out_features: int, in_features: int) -> int:
+    """The parts ``tq_linear`` computes a product of these sizes in."""
+    nbytes = int(_lib.lib().tq_linear_workspace_size(rows, out_features, in_features))
+    return max(1, nbytes // (4 * rows * out_features))
+
+
 def uses_rows_kernel(rows: int, out_features: int, in_features: int) -> bool:
     """Whether a linear layer of these sizes runs on ``tq_linear`` (else on the library GEMM)."""
+    if rows < ROWS_KERNEL_MIN_ROWS or in_features % 32 or in_features == 0:
+        return False
     tiles = ((rows + 127) >> 7) * ((out_features + 63) >> 6)
-    if rows < ROWS_KERNEL_MIN_ROWS:
+    if tiles >= ROWS_KERNEL_MIN_TILES:
+        return True
+    if in_features < SPLIT_MIN_K or rows < SPLIT_MIN_ROWS:
         return False
-    if tiles < ROWS_KERNEL_MIN_TILES and (in_features < SPLIT_MIN_K or rows < SPLIT_MIN_ROWS
-                                          or tiles > SPLIT_MAX_TILES or out_features % 4):  # fmt: skip
-        return False
-    return in_features % 32 == 0 and in_features > 0
+    return _split_parts(rows, out_features, in_features) * tiles >= ROWS_KERNEL_MIN_TILES
 
 
 def _saves_host_time(rows: int, out_features: int, in_features: int) -> bool:
