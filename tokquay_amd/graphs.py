@@ -177,8 +177,7 @@ class DecodeGraphs:
         tokens = s.tokens.clone()  # the warm-up runs overwrite what this step's source rows read
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
-        # Warm-up launches of what is captured (same inputs: the K/V writes are idempotent).
-        with torch.cuda.stream(side), ops.captured_form():
+        with torch.cuda.stream(side):  # warm-up launches (same inputs: the K/V writes are idempotent)
             for _ in range(2):
                 self._forward(rows, ids_only)
                 s.tokens.copy_(tokens)
