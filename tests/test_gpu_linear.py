@@ -157,6 +157,9 @@ def test_calls_the_kernel_does_not_take_run_as_before(monkeypatch):
                                    atol=1e-4)  # fmt: skip
         half = torch.nn.Linear(64, 2304).cuda().half()
         assert ops.linear(x.half(), half).dtype == torch.half
+        for dtype in (torch.half, torch.bfloat16):
+            with torch.autocast("cuda", dtype=dtype):
+                assert ops.linear(x, lin).dtype == ops.lm_head(x, lin.weight).dtype == dtype
         assert not taken
         ops.linear(x, lin)
         assert len(taken) == 1

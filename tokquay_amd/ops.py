@@ -579,7 +579,9 @@ def uses_rows_kernel(rows: int, out_features: int, in_features: int) -> bool:
 def _rows_kernel_takes(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None) -> bool:
     """Whether ``x @ w.T + bias`` goes to ``tq_linear``: by its sizes (``uses_rows_kernel``), for plain
     float32 tensors on one HIP device in the layout it reads, and if nothing must see torch's own
-    product (a gradient, a functorch transform, forward-mode AD, a tensor subclass)."""
+    product (a gradient, a functorch transform, forward-mode AD, a tensor subclass, autocast)."""
+    if torch.is_autocast_enabled("cuda"):  # torch's products return the autocast type
+        return False
     n, k = w.shape
     if x.dim() != 2 or x.size(1) != k:
         return False
