@@ -13,6 +13,9 @@ import sys
 
 import pytest
 import torch
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.overrides import TorchFunctionMode
+from torch.utils.flop_counter import FlopCounterMode
 
 from tokquay_amd import _lib, ops
 
@@ -163,6 +166,39 @@ def test_calls_the_kernel_does_not_take_run_as_before(monkeypatch):
         assert not taken
         ops.linear(x, lin)
         assert len(taken) == 1
+
+
+class _Names(TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.seen = [*getattr(self, "seen", []), getattr(func, "__name__", "")]
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [100, 800])
+def test_tracers_and_modes_see_torch_products(rows):
+    """A traced or recorded layer holds torch's own product, and runs on other sizes and strides."""
+    lin = torch.nn.Linear(3072, 768).cuda().requires_grad_(False)
+    x = torch.randn(rows, 3072, device="cuda")
+    f = lambda t: ops.linear(t, lin)  # noqa: E731
+    assert ops._rows_kernel_takes(x, lin.weight, lin.bias)
+    with torch.device("cuda"):
+        assert ops._rows_kernel_takes(x, lin.weight, lin.bias)
+    others = [x, x[: rows - 1], torch.randn(rows, 6144, device="cuda")[:, ::2], torch.randn(3072, 130, device="cuda").t()]
+    same = lambda got, t: torch.testing.assert_close(got, torch.addmm(lin.bias, t, lin.weight.t()), rtol=1e-4, atol=1e-4)  # noqa: E731
+    traced = torch.jit.trace(f, (x,), check_trace=False)
+    recorded = make_fx(f)(x)
+    assert [n.target for n in recorded.graph.nodes if "addmm" in str(n.target)] == [torch.ops.aten.addmm.default]
+    compiled = torch.compile(f, backend="eager", fullgraph=True)
+    for t in others:
+        same(traced(t), t), same(recorded(t), t), same(compiled(t), t)
+    torch._dynamo.reset()
+    with FlopCounterMode(display=False) as flops:
+        f(x)
+    assert flops.get_total_flops() == 2 * rows * 3072 * 768
+    with _Names() as names:
+        f(x)
+    assert "addmm" in names.seen
 
 
 @pytest.mark.gpu

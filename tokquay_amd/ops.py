@@ -20,6 +20,7 @@ import functools
 import math
 
 import torch
+from torch.utils._device import DeviceContext
 
 from tokquay_amd import _lib, torch_ops
 
@@ -576,11 +577,22 @@ def uses_rows_kernel(rows: int, out_features: int, in_features: int) -> bool:
     return _split_parts(rows, out_features, in_features) * tiles >= ROWS_KERNEL_MIN_TILES
 
 
+def _recorded() -> bool:
+    """Whether a tracer or a mode (FX, jit.trace, torch.compile, a flop counter, ...) sees torch's calls: a
+    recorded program runs on other sizes and layouts than those the kernel's rule looked at. The mode
+    behind ``with torch.device(...)`` only makes new tensors."""
+    if torch.compiler.is_compiling() or torch._C._is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
+        return True
+    modes = range(torch._C._len_torch_function_stack())
+    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in modes)
+
+
 def _rows_kernel_takes(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None) -> bool:
     """Whether ``x @ w.T + bias`` goes to ``tq_linear``: by its sizes (``uses_rows_kernel``), for plain
     float32 tensors on one HIP device in the layout it reads, and if nothing must see torch's own
-    product (a gradient, a functorch transform, forward-mode AD, a tensor subclass, autocast)."""
-    if torch.is_autocast_enabled("cuda"):  # torch's products return the autocast type
+    product (a gradient, a functorch transform, forward-mode AD, a tensor subclass, autocast, a tracer
+    or mode)."""
+    if _recorded() or torch.is_autocast_enabled("cuda"):  # torch's products return the autocast type
         return False
     n, k = w.shape
     if x.dim() != 2 or x.size(1) != k:
