@@ -257,10 +257,12 @@ __global__ __launch_bounds__(kWave* WM, WM == 8 ? 1 : 2) void linear_kernel(cons
   const int oc = 4 * (lane & 7);
 #pragma unroll
   for (int n = 0; n < NB; ++n) {
+    wave_lds_fence();  // after the reads of the block before
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       *reinterpret_cast<floatx4*>(&s.out.rows[wave][i][8 * r + 4 * g]) =
           floatx4{acc[n][4 * r], acc[n][4 * r + 1], acc[n][4 * r + 2], acc[n][4 * r + 3]};
+    wave_lds_fence();
     const int c = n0 + 32 * n + oc;
     floatx4 b = {0.f, 0.f, 0.f, 0.f};
     if (a.bias != nullptr) {

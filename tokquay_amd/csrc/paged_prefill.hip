@@ -197,11 +197,13 @@ __device__ __forceinline__ constexpr int pair_row(int place) { return 4 * (place
 // 16 r + (c ^ r): neither side has bank conflicts.
 template <bool PAIR>
 __device__ __forceinline__ void place_k(float4* slots, int j, int g, const float (&kreg)[16], float (&kout)[16]) {
+  wave_lds_fence();  // after the reads of the tile before
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int r = 4 * t + g;
     slots[16 * r + (j ^ r)] = make_float4(kreg[4 * t], kreg[4 * t + 1], kreg[4 * t + 2], kreg[4 * t + 3]);
   }
+  wave_lds_fence();
   const int row = PAIR ? pair_row(j) : j;
 #pragma unroll
   for (int v = 0; v < 4; ++v) {

@@ -71,6 +71,13 @@ __device__ __forceinline__ float row16_sum(float v) {
   return v;
 }
 
+// Between one lane's LDS accesses and those of the other lanes of its wave to the same words: the LDS takes
+// a wave's accesses in program order, and this keeps the compiler to it. No instruction.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ void flag_error(int32_t* d_error, int bits) {
   if (d_error != nullptr) atomicOr(d_error, bits);
 }
