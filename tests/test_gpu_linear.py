@@ -95,6 +95,27 @@ def test_non_finite_inputs_follow_fp32():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(200, 160, 128), (1000, 2304, 768), (1987, 2304, 96), (640, 768, 3072)])
+def test_non_finite_rows_leave_the_others_alone(m, n, k):
+    """The rows and columns without an infinity or NaN keep their bits; those with one follow fp32."""
+    x, w, b = _inputs(m, n, k)
+    clean = ops._rows_linear(x, w, b, True)
+    rows, cols = [3, 34, 35, 130, m - 1], [0, 33, n - 1]
+    for i, r in enumerate(rows):
+        x[r, (7 * i) % k] = [float("inf"), float("nan"), float("-inf"), 3.4e38, float("nan")][i]
+    for i, c in enumerate(cols):
+        w[c, (11 * i + 5) % k] = [float("nan"), float("inf"), float("-inf")][i]
+    got = ops._rows_linear(x, w, b, True)
+    keep = torch.ones(m, n, dtype=torch.bool, device="cuda")
+    keep[rows], keep[:, cols] = False, False
+    assert torch.equal(got[keep], clean[keep])
+    ref = torch.nn.functional.gelu(torch.addmm(b.double(), x.double(), w.double().t()).float(), approximate="tanh")
+    assert torch.equal(got.isnan(), ref.isnan())
+    fin = ref.isfinite()
+    torch.testing.assert_close(got[fin], ref[fin], rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.gpu
 def test_parts_of_k_follow_fp32_and_need_their_workspace():
     x, w, b = _inputs(130, 512, 1024)
     x[5, 700], w[9, 3] = float("inf"), float("nan")

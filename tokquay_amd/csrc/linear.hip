@@ -16,9 +16,9 @@
 // fp32 and split on the way in, nothing is kept between calls.
 //
 // Infinities, NaN and overflow: the split of a non-finite number (or of one that rounds past
-// the largest bf16) is NaN, so every output it touches comes out non-finite. A wave that sees
-// a non-finite accumulator computes its outputs again with plain fp32 FMAs, which gives them
-// IEEE's value.
+// the largest bf16) is NaN, so every output it touches comes out non-finite. Outputs whose
+// accumulator is not finite, and no others, are computed again with plain fp32 FMAs, which give
+// them IEEE's value: the wave's lanes share one output's K (row_dot).
 //
 // Work split: a workgroup of WM waves covers 32 WM rows x 32 NB columns; wave w owns rows
 // 32 w .. 32 w + 31 and all the columns, as NB accumulators of v_mfma_f32_32x32x16_bf16 (A = W,
@@ -47,6 +47,8 @@
 //
 // Reference semantics: nn.Linear (tokquay/model.py:62-63, :103-104), the tanh GELU (:107), the
 // tied LM head (:180-181).
+
+#include <float.h>
 
 #include <type_traits>
 
@@ -87,6 +89,21 @@ __device__ __forceinline__ float gelu(float v) {
 __device__ __forceinline__ void load8(const __amdgpu_buffer_rsrc_t& d, floatx4 (&r)[2], uint32_t offset, int32_t k) {
   r[0] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(d, offset, k * 4, 0));
   r[1] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(d, offset + 16, k * 4, 0));
+}
+
+// sum_k x[k] w[k] in fp32, K in whole steps, by one wave: the lanes take four k at a time and their sums are added
+// pairwise. Every lane returns the sum.
+__device__ __forceinline__ float row_dot(const float* x, const float* w, int32_t K) {
+  const int lane = threadIdx.x & (kWave - 1);
+  float v = 0.f;
+  for (int32_t k = 4 * lane; k < K; k += 4 * kWave) {
+    const floatx4 xv = *reinterpret_cast<const floatx4*>(x + k), wv = *reinterpret_cast<const floatx4*>(w + k);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v = fmaf(xv[e], wv[e], v);
+  }
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  return v;
 }
 
 template <int WM, int NB, int DEPTH>
@@ -238,20 +255,8 @@ __global__ __launch_bounds__(kWave* WM, WM == 8 ? 1 : 2) void linear_kernel(cons
   for (int n = 0; n < NB; ++n)
 #pragma unroll
     for (int r = 0; r < 16; ++r) probe = fmaf(acc[n][r], 0.f, probe);
-  const bool plain = __builtin_amdgcn_ballot_w64(probe != probe) != 0;  // uniform: see the top of the file
+  const bool redo = __builtin_amdgcn_ballot_w64(probe != probe) != 0;  // uniform: see the top of the file
   __syncthreads();  // the stage buffers become the output blocks
-  if (plain) {
-    for (int e = lane; e < 32 * BN; e += kWave) {
-      const int m = m0 + e / BN, c = n0 + e % BN;
-      if (m >= a.M || c >= a.N) continue;
-      const float* xp = a.x + (int64_t)m * a.x_stride + k_lo;
-      const float* wp = a.w + (int64_t)c * a.K + k_lo;
-      float v = 0.f;
-      for (int k = 0; k < a.k_part; ++k) v = fmaf(xp[k], wp[k], v);
-      y[(int64_t)m * a.y_stride + c] = finish(a.bias != nullptr ? v + a.bias[c] : v);
-    }
-    return;
-  }
   // Each 32 x 32 block goes through the wave's own LDS rows, so that the stores cover whole
   // 128-byte runs of y (lane: row 8 t + lane / 8, columns 4 (lane % 8) ..).
   const int oc = 4 * (lane & 7);
@@ -262,6 +267,21 @@ __global__ __launch_bounds__(kWave* WM, WM == 8 ? 1 : 2) void linear_kernel(cons
     for (int r = 0; r < 4; ++r)
       *reinterpret_cast<floatx4*>(&s.out.rows[wave][i][8 * r + 4 * g]) =
           floatx4{acc[n][4 * r], acc[n][4 * r + 1], acc[n][4 * r + 2], acc[n][4 * r + 3]};
+    if (redo) {
+#pragma unroll 1
+      for (int r = 0; r < 16; ++r) {
+        float& v = s.out.rows[wave][i][8 * (r / 4) + 4 * g + r % 4];  // row m0 + i, column col(g)
+        const auto col = [&](int group) { return n0 + 32 * n + 8 * (r / 4) + 4 * group + r % 4; };
+        uint64_t todo = __builtin_amdgcn_ballot_w64(!(fabsf(v) <= FLT_MAX) && m0 + i < a.M && col(g) < a.N);
+        while (todo != 0) {  // uniform
+          const int from = __builtin_ctzll(todo);
+          todo &= todo - 1;
+          const float dot = row_dot(a.x + (int64_t)(m0 + (from & 31)) * a.x_stride + k_lo,
+                                    a.w + (int64_t)col(from >> 5) * a.K + k_lo, a.k_part);
+          if (lane == from) v = dot;
+        }
+      }
+    }
     wave_lds_fence();
     const int c = n0 + 32 * n + oc;
     floatx4 b = {0.f, 0.f, 0.f, 0.f};
