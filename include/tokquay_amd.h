@@ -345,9 +345,12 @@ tq_status tq_argmax_rows(int64_t* out, const float* logits, int64_t num_rows, in
  * x is M rows of K floats (row stride x_stride elements), W is [N, K] contiguous, bias (may be
  * null) has N entries, y is M rows of N floats (row stride y_stride). epilogue: 0 = none, 1 =
  * tanh-form GELU. fp32 in, fp32 out, at fp32's precision (each operand split into three bf16
- * numbers that add up to it, the products accumulated in fp32); infinities and NaN give what
- * fp32 arithmetic gives. K a multiple of 32, at most 2^21; x and W 16-byte aligned, x_stride a
- * multiple of 4 (y and bias: any alignment). Outputs must not alias inputs.
+ * numbers that add up to it, the products accumulated in fp32). Infinities and NaN give what fp32
+ * arithmetic gives, and so do operands below 2^-110, of which the split loses bits, unless they
+ * meet operands above 2^32 and no output of the tile (32 rows x 32-128 columns) is above 2^32: an
+ * output is then off by up to 2^-134 of the operand each meets. K a multiple of 32, below 2^21; x and
+ * W 16-byte aligned, x_stride a multiple of 4 (y and bias: any alignment). Outputs must not alias
+ * inputs.
  *
  * Replaces nn.Linear over the packed rows of a prefill step (tokquay/model.py:62-63, :103-107)
  * and the tied LM head of a large batch (:180-181).

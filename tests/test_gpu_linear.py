@@ -32,7 +32,8 @@ def _check(got, x, w, b, gelu=False):
     if gelu:
         bound = 1.13 * bound + 16 * EPS * (1 + ref.abs())
         ref = torch.nn.functional.gelu(ref, approximate="tanh")
-    assert ((got - ref).abs() <= bound + 1e-30).all(), float(((got - ref).abs() - bound).max())
+    bound = bound + x.size(1) * 2.0**-149  # subnormal products
+    assert ((got - ref).abs() <= bound).all(), float(((got - ref).abs() - bound).max())
 
 
 def _inputs(m, n, k, bias=True, seed=0):
@@ -70,15 +71,34 @@ def test_strided_rows_and_unaligned_outputs():
 
 @pytest.mark.gpu
 def test_wide_ranges_stay_fp32():
-    """Rows and weights from 1e-30 to 1e30 keep fp32's precision (the limbs have fp32's exponents)."""
+    """Rows from 1e-44 to 1e15 against weights from 1e-5 to 1e18 keep fp32's precision, those included whose limbs
+    run out of exponents."""
     x, w, _ = _inputs(160, 96, 256, bias=False)
-    x = x * torch.logspace(-30, 15, 160).cuda()[:, None]
+    x = x * torch.logspace(-44, 15, 160, dtype=torch.double).cuda()[:, None]
     w = w * torch.logspace(-5, 18, 96).cuda()[:, None]
+    x = x.float()
     _check(ops._rows_linear(x, w, None, False), x, w, None)
-    eye = torch.eye(256, device="cuda")
-    y = ops._rows_linear(x, eye, None, False)
-    big = x.abs() > 1e-25  # the limbs of smaller values fall below the smallest normal number
-    assert torch.equal(y[big], x[big])
+    assert torch.equal(ops._rows_linear(x, torch.eye(256, device="cuda"), None, False), x)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(70, 100, 96), (1000, 2304, 768), (300, 768, 3072)])
+def test_tiny_operands(m, n, k):
+    """Tiny operands among ordinary ones, alone in their row, behind huge partners, and as weights; rows and
+    columns of zeros give zeros."""
+    x, w, _ = _inputs(m, n, k, bias=False)
+    x[1], x[2], x[33], x[m - 1] = x[1] * 1e-36, x[2] * 1e-41, 0.0, 0.0
+    x[3, ::2] *= 1e-38
+    x[m - 1, k - 1], x[0, 1] = 3e-39, 2e-36
+    w[n - 1], w[5], w[6] = 0.0, w[5] * 1e-37, 0.0
+    w[7, k - 1], w[6, 1] = 1e30, 1e33  # one product each: x's tiny elements times these
+    got = ops._rows_linear(x, w, None, False)
+    _check(got, x, w, None)
+    assert (got[33] == 0).all() and (got[:, n - 1] == 0).all()
+    others = torch.ones(m, n, dtype=torch.bool, device="cuda")
+    others[[1, 2, 3, 33, m - 1, 0]], others[:, [5, 6, 7, n - 1]] = False, False
+    clean, weights, _ = _inputs(m, n, k, bias=False)
+    assert torch.equal(got[others], ops._rows_linear(clean, weights, None, False)[others])
 
 
 @pytest.mark.gpu

@@ -32,6 +32,16 @@ __device__ __forceinline__ void split8(const floatx4& lo, const floatx4& hi, uin
   }
 }
 
+// The limbs of |v| >= kWhole add up to v; those of a smaller v are off by at most 2^-134, half the smallest bf16
+// (the conversion and the MFMA keep bf16 subnormals). An output summed over n products x w is then off by
+// at most n 2^-133 max(|x|, |w|).
+constexpr float kWhole = 0x1p-110f;
+
+// Whether 0 < |v| < kWhole.
+__device__ __forceinline__ bool loses_bits(float v) {
+  return 2 * __float_as_uint(v) - 1 < 2 * __builtin_bit_cast(uint32_t, kWhole) - 1;  // 0 wraps to the largest
+}
+
 // The six limb products that make an fp32 product, smallest first: limb of A, limb of B.
 constexpr int kLimbA[6] = {2, 0, 1, 1, 0, 0}, kLimbB[6] = {0, 2, 1, 0, 1, 0};
 
