@@ -85,21 +85,25 @@ def test_dispatch_order_keeps_the_bits_and_bad_metadata_is_reported():
 
 @pytest.mark.gpu
 def test_non_finite_keys_follow_fp32_softmax():
-    """An infinite key gives a query that sees it what fp32 softmax gives (NaN, or no weight), and does
-    not reach the queries before it."""
+    """An infinite key gives a query that sees it what fp32 softmax gives (NaN, or no weight), and the queries
+    and heads that do not see it keep their bits, those of the same wave too."""
     starts, lens = SHAPES[0]
     sc = Scenario(starts, lens, n_head=H)
     sc.k[0, 3, 100, 7] = float("inf")
     sc.k[2, 5, 40, 0] = float("-inf")
     pool, out, batch = sc.run_product()
     clean, want, _ = Scenario(starts, lens, n_head=H).run_product()
+    unseen = torch.ones(want.size(0), H, dtype=torch.bool)
+    same = want.view(-1, H, 64)
     want = want.double().view(-1, H, 64).clone()
     at = [0, 256, 456, 585, 713]
     for b, h, pos in ((0, 3, 100), (2, 5, 40)):
         q, k, v = (t[b, h].double() for t in (sc.q, sc.k, sc.v))
+        unseen[at[b] + pos : at[b] + lens[b], h] = False
         for t in range(pos, lens[b]):
             p = torch.softmax(k[: t + 1] @ q[t] / math.sqrt(64), 0)
             want[at[b] + t, h] = p @ v[: t + 1]
     got = out.double().view(-1, H, 64)
+    assert torch.equal(out.view(-1, H, 64)[unseen], same[unseen])
     assert want.isnan().any() and want[at[0] + 100 : at[0] + 256, 3].isfinite().any()
     torch.testing.assert_close(got, want, rtol=RTOL, atol=ATOL, equal_nan=True)

@@ -25,9 +25,9 @@
 // rate a large bf16 library product reaches here, a sixth each. Three per CU (168 VGPRs) spill and
 // ran 10 % slower.
 //
-// The softmax is the 16-row kernels' (log2 units, lazy maximum). A wave whose result is not
-// finite computes it again from the fp32 values (limbs of infinities and NaN are NaN, which
-// would also reach queries that must not see them).
+// The softmax is the 16-row kernels' (log2 units, lazy maximum). Queries whose result is not finite, and no
+// others, are computed again from the fp32 values (limbs of infinities and NaN are NaN, which would
+// also reach queries that must not see them).
 #pragma once
 
 #include <float.h>
@@ -310,19 +310,24 @@ __global__ __launch_bounds__(kWave* kWideWaves, 2) void prefill_wide_kernel(cons
   float probe = l * 0.f;
 #pragma unroll
   for (int r = 0; r < 16; ++r) probe = fmaf(o[0][r], 0.f, fmaf(o[1][r], 0.f, probe));
-  if (__builtin_amdgcn_ballot_w64(probe != probe) != 0) {  // uniform
-    for (int r = 0; r < rows; ++r) prefill_plain_row<BS>(a, bt, head_base, row0 + q0 + r, start + q0 + r, h);
-    return;
+  // Lanes i and i + 32 hold the two dim blocks of query i.
+  const uint64_t lanes = __builtin_amdgcn_ballot_w64(probe != probe && i < rows);
+  uint32_t again = (uint32_t)lanes | (uint32_t)(lanes >> 32);  // uniform: queries to compute again
+  if (i < rows && !(again >> i & 1)) {
+    const float inv = 1.f / l;
+    float* op = a.out + (int64_t)(row0 + q0 + i) * a.out_stride + h * kHeadDim;
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<floatx4*>(op + 32 * d + 8 * r + 4 * g) =
+            floatx4{o[d][4 * r], o[d][4 * r + 1], o[d][4 * r + 2], o[d][4 * r + 3]} * inv;
   }
-  if (i >= rows) return;
-  const float inv = 1.f / l;
-  float* op = a.out + (int64_t)(row0 + q0 + i) * a.out_stride + h * kHeadDim;
-#pragma unroll
-  for (int d = 0; d < 2; ++d)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      *reinterpret_cast<floatx4*>(op + 32 * d + 8 * r + 4 * g) =
-          floatx4{o[d][4 * r], o[d][4 * r + 1], o[d][4 * r + 2], o[d][4 * r + 3]} * inv;
+  while (again != 0) {
+    const int r = __builtin_ctz(again);
+    again &= again - 1;
+    prefill_plain_row<BS>(a, bt, head_base, row0 + q0 + r, start + q0 + r, h);
+  }
 }
 
 }  // namespace
