@@ -107,3 +107,37 @@ def test_non_finite_keys_follow_fp32_softmax():
     assert torch.equal(out.view(-1, H, 64)[unseen], same[unseen])
     assert want.isnan().any() and want[at[0] + 100 : at[0] + 256, 3].isfinite().any()
     torch.testing.assert_close(got, want, rtol=RTOL, atol=ATOL, equal_nan=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bs", [16, 32])
+def test_tiny_operands_keep_fp32(bs):
+    """Values below 2^-110, whose limbs do not add up to them, and tiny queries against huge keys (and the
+    reverse) give what fp32 gives, dims of zeros give zeros; heads without any keep their bits."""
+    starts, lens = SHAPES[1]
+    sc = Scenario(starts, lens, block_size=bs, n_head=H)
+    _, clean, _ = Scenario(starts, lens, block_size=bs, n_head=H).run_product()
+    for h, scale in ((3, 1e-34), (17, 1e-36), (40, 1e-39)):
+        sc.v[:, h] *= scale
+        for b, s in enumerate(starts):
+            for p in range(s):
+                sc.pool[sc.tables[b][p // bs], 0, 1, h, p % bs] *= scale
+    sc.v[:, 5, ::2, :7] = 0.0
+    for h, scale in ((20, 1e34), (50, 1e-34)):
+        sc.q[:, h] *= scale
+        sc.k[:, h] /= scale
+        for b, s in enumerate(starts):
+            for p in range(s):
+                sc.pool[sc.tables[b][p // bs], 0, 0, h, p % bs] /= scale
+    pool, out, batch = sc.run_product()
+    same = [h for h in range(H) if h not in (3, 5, 17, 20, 40, 50)]
+    got = out.view(-1, H, 64)
+    assert torch.equal(got[:, same], clean.view(-1, H, 64)[:, same])
+    at = 0
+    for want in sc.brute_force(pool):
+        have = got[at : at + want.shape[0]].double()
+        want = torch.from_numpy(want)
+        for h, scale in ((3, 1e-34), (5, 1.0), (17, 1e-36), (20, 1.0), (40, 1e-39), (50, 1.0)):
+            err = (have[:, h] - want[:, h]).abs().max()
+            assert err <= 1e-5 * scale + 2.0**-140, (h, float(err))  # 2^-140: subnormal products of fp32
+        at += want.shape[0]

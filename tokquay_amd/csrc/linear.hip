@@ -102,14 +102,6 @@ __device__ __forceinline__ void load8(const __amdgpu_buffer_rsrc_t& d, floatx4 (
   r[1] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(d, offset + 16, k * 4, 0));
 }
 
-// NaN if any is (v_minimum3_f32, v_maximum3_f32).
-__device__ __forceinline__ float min3(float a, float b, float c) {
-  return __builtin_elementwise_minimum(__builtin_elementwise_minimum(a, b), c);
-}
-__device__ __forceinline__ float max3(float a, float b, float c) {
-  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
-}
-
 // sum_k x[k] w[k] in fp32, K in whole steps, by one wave: the lanes take four k at a time and their sums are added
 // pairwise. Every lane returns the sum.
 __device__ __forceinline__ float row_dot(const float* x, const float* w, int32_t K) {

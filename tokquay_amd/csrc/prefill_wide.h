@@ -25,9 +25,13 @@
 // rate a large bf16 library product reaches here, a sixth each. Three per CU (168 VGPRs) spill and
 // ran 10 % slower.
 //
-// The softmax is the 16-row kernels' (log2 units, lazy maximum). Queries whose result is not finite, and no
-// others, are computed again from the fp32 values (limbs of infinities and NaN are NaN, which would
-// also reach queries that must not see them).
+// The softmax is the 16-row kernels' (log2 units, lazy maximum). Queries whose result is not finite are
+// computed again from the fp32 values (limbs of infinities and NaN are NaN, which would also reach queries
+// that must not see them), and so are those that values of V below 2^-110 cost precision: each is off by up to 2^-134
+// (split_bf16.h), as is each probability, which is below 2^-22 of an output of 2^-112 (keys max |v| + 1). A wave with an
+// output below keys 2^-80 or above 2^32 looks through its V for such values and the largest one. All other
+// queries keep their bits. Queries and keys: a score is off by up to 64 x 2^-133 of the larger operand, under
+// 2^-20 up to 2^107. (Largest |K| and |V| kept in the loop, for outputs of every size, took 2-6 %.)
 #pragma once
 
 #include <float.h>
@@ -63,6 +67,31 @@ __device__ __forceinline__ void prefill_plain_row(const PrefillArgs& a, const in
     m = mn;
   }
   a.out[(int64_t)row * a.out_stride + h * kHeadDim + lane] = o / l;
+}
+
+// Whether the first n keys' V of one head hold a value that loses bits, and the largest finite |v|. By one wave.
+template <int BS>
+__device__ __forceinline__ bool values_lose_bits(const PrefillArgs& a, const int32_t* bt, const float* head_base, int n,
+                                                 float& largest) {
+  const int lane = threadIdx.x & (kWave - 1);
+  bool loses = false;
+  float m = 0.f;
+#pragma unroll 4
+  for (int key = lane >> 4; key < n; key += 4) {  // 16 lanes a row
+    const int32_t blk = bt[key / BS];
+    if ((uint32_t)blk >= (uint32_t)a.num_blocks) continue;
+    const floatx4 v = *reinterpret_cast<const floatx4*>(head_base + (int64_t)blk * a.block_stride + a.kv_stride +
+                                                        (key % BS) * kHeadDim + 4 * (lane & 15));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      loses |= loses_bits(v[e]);
+      m = fabsf(v[e]) <= FLT_MAX ? fmaxf(m, fabsf(v[e])) : m;
+    }
+  }
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+  largest = m;
+  return __builtin_amdgcn_ballot_w64(loses) != 0;
 }
 
 template <int BS>
@@ -307,11 +336,21 @@ __global__ __launch_bounds__(kWave* kWideWaves, 2) void prefill_wide_kernel(cons
 
   const auto other = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
   l = __uint_as_float(other[0]) + __uint_as_float(other[1]);
-  float probe = l * 0.f;
+  float least = FLT_MAX, most = l;  // of the query's |sums| in this lane; NaN if any is
 #pragma unroll
-  for (int r = 0; r < 16; ++r) probe = fmaf(o[0][r], 0.f, fmaf(o[1][r], 0.f, probe));
+  for (int r = 0; r < 16; ++r) {
+    least = min3(least, fabsf(o[0][r]), fabsf(o[1][r]));
+    most = max3(most, fabsf(o[0][r]), fabsf(o[1][r]));
+  }
+  bool redo = !(most <= FLT_MAX);
+  // Uniform: whether values may have lost bits (see the top of the file).
+  if (__builtin_amdgcn_ballot_w64(!redo && (least < (float)kend * 0x1p-80f || most > 0x1p32f)) != 0) {
+    float vmax;
+    if (values_lose_bits<BS>(a, bt, head_base, kend, vmax))
+      redo |= least < 0x1p-112f * fmaf((float)kend, vmax, l);
+  }
   // Lanes i and i + 32 hold the two dim blocks of query i.
-  const uint64_t lanes = __builtin_amdgcn_ballot_w64(probe != probe && i < rows);
+  const uint64_t lanes = __builtin_amdgcn_ballot_w64(redo && i < rows);
   uint32_t again = (uint32_t)lanes | (uint32_t)(lanes >> 32);  // uniform: queries to compute again
   if (i < rows && !(again >> i & 1)) {
     const float inv = 1.f / l;

@@ -42,6 +42,14 @@ __device__ __forceinline__ bool loses_bits(float v) {
   return 2 * __float_as_uint(v) - 1 < 2 * __builtin_bit_cast(uint32_t, kWhole) - 1;  // 0 wraps to the largest
 }
 
+// NaN if any is (v_minimum3_f32, v_maximum3_f32).
+__device__ __forceinline__ float min3(float a, float b, float c) {
+  return __builtin_elementwise_minimum(__builtin_elementwise_minimum(a, b), c);
+}
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
+}
+
 // The six limb products that make an fp32 product, smallest first: limb of A, limb of B.
 constexpr int kLimbA[6] = {2, 0, 1, 1, 0, 0}, kLimbB[6] = {0, 2, 1, 0, 1, 0};
 
