@@ -222,10 +222,13 @@ __device__ __forceinline__ void place_k(float4* slots, int j, int g, const float
 // loop: with the pipelined one (126 VGPRs, its decode workgroups still at 4 waves per SIMD) the
 // steps of four 256-token prompt chunks beside 128 decoding sequences ran from 3 % faster to 2 %
 // slower depending on the chunk.
-template <int BS_CT, int KS, int QH = 1, bool PIPE = (BS_CT > 0)>
+// PLACE: K tiles through place_k() (load_kv_block_tile).
+template <int BS_CT, int KS, int QH, bool PIPE, bool PLACE>
 __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int dispatch) {
   static_assert(BS_CT == 0 || BS_CT == 8 || BS_CT % kTile == 0, "a key tile lies in one block, or is two");
   static_assert(!PIPE || BS_CT > 0, "the pipelined key loop reads whole blocks");
+  static_assert(!PLACE || BS_CT > 0, "only whole tiles are placed");
+  static_assert(PLACE || BS_CT != 8, "a block pair's K rows are not the lanes'");
   static_assert(QH == 1 || KS == 1, "two query tiles per wave only without a key split");
   const int lane = threadIdx.x & (kWave - 1);
   // Wave-uniform by construction; readfirstlane lets the compiler keep the key-tile loop
@@ -342,11 +345,10 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
   // lane's test fires), max as v_maximum3_f32 (no operand canonicalization), and one ballot
   // for all of the wave's query tiles.
   constexpr bool kPair = BS_CT == 8;
-  constexpr bool kPlaceK = BS_CT > 0 && (KS > 1 || !PIPE || kPair);
-  __shared__ float4 s_k[KS][kPlaceK ? kTile * kHeadDim / 4 : 1];
+  __shared__ float4 s_k[KS][PLACE ? kTile * kHeadDim / 4 : 1];
   auto consume = [&](int kt, const float (&kload)[16], const float4 (&vreg)[4]) {
       float kreg[16];
-      if constexpr (kPlaceK) {
+      if constexpr (PLACE) {
         place_k<kPair>(s_k[wave], j, g, kload, kreg);
       } else {
   #pragma unroll
@@ -421,7 +423,7 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
       load_kv_block_pair(a, head_base, __builtin_amdgcn_readlane(tb_id, at), __builtin_amdgcn_readlane(tb_id, at + 1),
                          kt, kend, j, g, kreg, vreg);
     else if constexpr (BS_CT > 0)
-      load_kv_block_tile<BS_CT, kPlaceK>(a, head_base, __builtin_amdgcn_readlane(tb_id, at), kt, kend, j, g, kreg,
+      load_kv_block_tile<BS_CT, PLACE>(a, head_base, __builtin_amdgcn_readlane(tb_id, at), kt, kend, j, g, kreg,
                                          vreg);
   };
 
@@ -574,9 +576,9 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
   }
 }
 
-template <int BS_CT, int KS, int QH = 1>
+template <int BS_CT, int KS, int QH, bool PLACE>
 __global__ __launch_bounds__(kWave* KS) void prefill_kernel(const PrefillArgs a) {
-  prefill_workgroup<BS_CT, KS, QH>(a, blockIdx.x);
+  prefill_workgroup<BS_CT, KS, QH, (BS_CT > 0), PLACE>(a, blockIdx.x);
 }
 
 // The 8-wave instance reserves this much extra (unused) LDS per workgroup so that a
@@ -586,13 +588,13 @@ __global__ __launch_bounds__(kWave* KS) void prefill_kernel(const PrefillArgs a)
 // tail chunk with 5 / 102 / 9 rows at position 768: 22.2 -> 14.5 us.
 constexpr size_t kLdsOneGroupPerCu = 64 * 1024;
 
-template <int BS_CT, int KS, int QH = 1>
+template <int BS_CT, int KS, int QH = 1, bool PLACE = (BS_CT == 8 || (BS_CT > 0 && KS > 1))>
 void launch_prefill_ks(const PrefillArgs& a, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
   const size_t lds = KS == 8 ? kLdsOneGroupPerCu : 0;
   if (start == nullptr && stop == nullptr)
-    hipLaunchKernelGGL((prefill_kernel<BS_CT, KS, QH>), dim3((unsigned)a.total), dim3(kWave * KS), lds, stream, a);
+    hipLaunchKernelGGL((prefill_kernel<BS_CT, KS, QH, PLACE>), dim3((unsigned)a.total), dim3(kWave * KS), lds, stream, a);
   else
-    hipExtLaunchKernelGGL((prefill_kernel<BS_CT, KS, QH>), dim3((unsigned)a.total), dim3(kWave * KS), lds, stream,
+    hipExtLaunchKernelGGL((prefill_kernel<BS_CT, KS, QH, PLACE>), dim3((unsigned)a.total), dim3(kWave * KS), lds, stream,
                           start, stop, 0, a);
 }
 
@@ -655,6 +657,22 @@ bool use_wide(const PrefillArgs& a) {
   return head_rows >= 1280 * 32 && 5 * head_rows >= 2 * held && (int64_t)a.max_blocks * a.block_size >= 256;
 }
 
+// Key-split launches place K through LDS, except where the tables hold at most two key tiles: there the trip
+// is longer than the loads it saves. Measured us (direct -> placed): prompts of 2 / 16 / 28 / 32 rows 4.2 / 4.1 /
+// 4.2 / 4.3 -> 4.5 / 4.3 / 4.4 / 4.4, eight of them 4.3 / 4.2 / 4.4 / 4.5 -> 4.6 / 4.4 / 4.6 / 4.6; tables of 48 / 64 / 112 keys
+// 4.6 / 4.8 / 5.6 -> 4.6 / 4.7 / 5.4. (Mixed launches always place: up to 2 % slower in some of those with tables below
+// 512 keys beside 64-128 decode rows, up to 8 % faster in others, 13-23 % faster at 956 keys.)
+template <int BS_CT, int KS>
+void launch_key_split(const PrefillArgs& a, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
+  if constexpr (BS_CT == 16 || BS_CT == 32) {
+    if ((int64_t)a.max_blocks * BS_CT <= 2 * kTile) {
+      launch_prefill_ks<BS_CT, KS, 1, false>(a, stream, start, stop);
+      return;
+    }
+  }
+  launch_prefill_ks<BS_CT, KS>(a, stream, start, stop);
+}
+
 template <int BS_CT>
 void launch_prefill(const PrefillArgs& a_in, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
   const int ks = choose_key_split((int64_t)a_in.groups * a_in.qtiles);
@@ -676,9 +694,9 @@ void launch_prefill(const PrefillArgs& a_in, hipStream_t stream, hipEvent_t star
         launch_prefill_ks<BS_CT, 1>(a, stream, start, stop);
       }
       break;
-    case 2: launch_prefill_ks<BS_CT, 2>(a, stream, start, stop); break;
-    case 4: launch_prefill_ks<BS_CT, 4>(a, stream, start, stop); break;
-    default: launch_prefill_ks<BS_CT, 8>(a, stream, start, stop); break;
+    case 2: launch_key_split<BS_CT, 2>(a, stream, start, stop); break;
+    case 4: launch_key_split<BS_CT, 4>(a, stream, start, stop); break;
+    default: launch_key_split<BS_CT, 8>(a, stream, start, stop); break;
   }
 }
 
@@ -809,7 +827,7 @@ __global__ __launch_bounds__(kWave* KS) void mixed_kernel(const PrefillArgs p, c
     decode_unit<DEC_BS, true>(d, rest / d.max_parts, u - rest * d.num_heads, rest % d.max_parts, lane);
     return;
   }
-  prefill_workgroup<PRE_BS, KS, 1, false>(p, idx);
+  prefill_workgroup<PRE_BS, KS, 1, false, (PRE_BS > 0)>(p, idx);
 }
 
 template <int DEC_BS, int PRE_BS, int KS>
