@@ -12,25 +12,31 @@ import torch
 
 from tests.paged_cases import ATOL, RTOL, Scenario
 from tokquay_amd import ops
-from tokquay_amd.kv_cache import PagedBatch
 
 H = 64
 SHAPES = [
     ([0, 0, 0, 0, 0], [256, 200, 129, 128, 97]),
     ([1000, 37, 300, 5], [300, 257, 31, 255]),
-    ([0, 64, 511, 15, 16], [385, 161, 160, 159, 2]),
+    ([0, 64, 511, 15, 16, 100], [385, 161, 160, 159, 2, 384]),
     ([3, 200, 31, 2000], [128, 127, 140, 250]),
 ]
 
 
-def _run_alone(sc, b):
-    """Sequence b's attention as a launch of its own (few rows: the 16-row kernels)."""
-    one = PagedBatch(sc.gpu_pool, sc.block_size, [sc.tables[b]], [sc.starts[b]], [sc.new_lens[b]])
-    rows = sc.rows[b]
-    out = torch.empty(len(rows), sc.C, device="cuda")
-    ops.paged_prefill(out, sc.qkv[rows, : sc.C], sc.gpu_pool, 0, one.prefill_block_tables, one.prefill_cu_seqlens,
-                      one.prefill_start, one.prefill_max_q)  # fmt: skip
-    return out
+# Relative 2-norm against float64: the six limb products measure 1e-7 to 4e-7 here; with the three largest only,
+# which RTOL and ATOL would let pass, it is 6e-6.
+NORM = 1e-6
+
+
+def _sixteen_row(sc, batch, pool):
+    """The same rows from the 16-row kernels: sequences without rows beside them leave 128-query workgroups
+    too empty to be taken, and change nothing else."""
+    qkv, B = sc.packed_qkv(batch.token_index).cuda(), len(sc.starts)
+    tables = torch.cat([batch.prefill_block_tables] + [batch.prefill_block_tables] * 2)
+    cu = torch.cat([batch.prefill_cu_seqlens, batch.prefill_cu_seqlens[-1:].expand(2 * B)]).contiguous()
+    start = torch.cat([batch.prefill_start, torch.zeros_like(batch.prefill_start).repeat(2)])
+    out = torch.empty(qkv.size(0), sc.C, device="cuda")
+    ops.paged_prefill(out, qkv[:, : sc.C], pool.cuda(), 0, tables, cu, start, batch.prefill_max_q)
+    return out.cpu()
 
 
 @pytest.mark.gpu
@@ -44,18 +50,22 @@ def test_matches_the_oracle(starts, lens, bs):
     torch.testing.assert_close(out, sc.packed_reference(out_ref, batch.token_index), rtol=RTOL, atol=ATOL)
     at = 0
     for want in sc.brute_force(pool_ref):
-        got = out[at : at + want.shape[0]].view(-1, H, 64)
-        torch.testing.assert_close(got.double(), torch.from_numpy(want), rtol=RTOL, atol=ATOL)
+        got, want = out[at : at + want.shape[0]].view(-1, H, 64).double(), torch.from_numpy(want)
+        torch.testing.assert_close(got, want, rtol=RTOL, atol=ATOL)
+        assert (got - want).norm() <= NORM * want.norm()
         at += want.shape[0]
-    # The launch is the wide one: its bits are not those of the sequences launched alone.
-    sc.gpu_pool, sc.qkv = pool.cuda(), sc.packed_qkv(batch.token_index).cuda()
-    cu = [0]
-    for n in lens:
-        cu.append(cu[-1] + n)
-    sc.rows = [torch.arange(cu[b], cu[b + 1], device="cuda") for b in range(len(lens))]
-    alone = torch.cat([_run_alone(sc, b) for b in range(len(lens))]).cpu()
-    torch.testing.assert_close(out, alone, rtol=RTOL, atol=ATOL)
-    assert not torch.equal(out, alone)
+    # The launch is the 128-query one: its bits are not those of the 16-row kernels.
+    other = _sixteen_row(sc, batch, pool)
+    torch.testing.assert_close(out, other, rtol=RTOL, atol=ATOL)
+    assert not torch.equal(out, other)
+
+
+@pytest.mark.gpu
+def test_too_few_rows_stay_on_the_16_row_kernels():
+    """What the check above rests on: a launch that is not well filled has the 16-row kernels' bits already."""
+    sc = Scenario([0, 64, 511, 15, 16], [385, 161, 160, 159, 2], n_head=H, seed=5)
+    pool, out, batch = sc.run_product()
+    assert torch.equal(out, _sixteen_row(sc, batch, pool))
 
 
 @pytest.mark.gpu
