@@ -8,9 +8,9 @@
 //   x w = x0 w0 + (x0 w1 + x1 w0) + (x0 w2 + x1 w1 + x2 w0) + terms below 2^-24 |x w|
 //
 // so six bf16 products, accumulated in fp32 by the MFMA, give the product to fp32's own
-// precision; the sum is the more exact for taking 16 k per accumulation instead of 4: against
-// float64, weights N(0, 0.02), rows N(0, 1): 2.1e-7 (K = 768) and 4.3e-7 (K = 3072) relative
-// where the fp32 MFMA GEMM of the library has 5.0e-7 and 9.9e-7. The fp32 MFMA peaks at 157
+// precision; the sum is a little more exact for taking 16 k per accumulation instead of 4: against
+// float64, weights N(0, 0.02), rows N(0, 1): 4.2e-7 (K = 768) and 8.6e-7 (K = 3072; 3.1e-7 to 4.3e-7 in
+// parts of K) relative where the fp32 MFMA GEMM of the library has 5.0e-7 and 9.9e-7. The fp32 MFMA peaks at 157
 // TFLOP/s on this GPU; bf16 runs ~1,200 (what a large library product reaches here, power
 // bound), a sixth of which is 200. The split costs no extra traffic: operands are read as
 // fp32 and split on the way in, nothing is kept between calls.

@@ -54,11 +54,10 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // Pointer to the first element of position `key` of this head's K tile (V is + kv_stride),
 // or nullptr when the block id is out of range.
-template <int BS_CT>
 __device__ __forceinline__ const float* key_row(const PrefillArgs& a, const int32_t* bt,
                                                 const float* head_base, int bs, int key) {
-  const int bi = BS_CT > 0 ? key / BS_CT : key / bs;
-  const int off = key - bi * (BS_CT > 0 ? BS_CT : bs);
+  const int bi = key / bs;
+  const int off = key - bi * bs;
   const int64_t blk = bt[bi];
   if ((uint64_t)blk >= (uint64_t)a.num_blocks) {
     flag_error(a.d_error, TQ_DEVERR_BLOCK_ID);
@@ -67,12 +66,11 @@ __device__ __forceinline__ const float* key_row(const PrefillArgs& a, const int3
   return head_base + blk * a.block_stride + (int64_t)off * kHeadDim;
 }
 
-template <int BS_CT>
 __device__ __forceinline__ void load_kv_tile(const PrefillArgs& a, const int32_t* bt, const float* head_base, int bs,
                                              int kt, int kend, int j, int g, float (&kreg)[16], float4 (&vreg)[4]) {
   {
     const int key = kt + j;
-    const float* p = key < kend ? key_row<BS_CT>(a, bt, head_base, bs, key) : nullptr;
+    const float* p = key < kend ? key_row(a, bt, head_base, bs, key) : nullptr;
     if (p != nullptr) {
       p += 16 * g;
 #pragma unroll
@@ -91,7 +89,7 @@ __device__ __forceinline__ void load_kv_tile(const PrefillArgs& a, const int32_t
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
     const int key = kt + 4 * g + s;
-    const float* p = key < kend ? key_row<BS_CT>(a, bt, head_base, bs, key) : nullptr;
+    const float* p = key < kend ? key_row(a, bt, head_base, bs, key) : nullptr;
     vreg[s] = p != nullptr ? *reinterpret_cast<const float4*>(p + a.kv_stride + 4 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
   }
 }
@@ -511,7 +509,7 @@ __device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int disp
         }
         load_tile(tb_id, ti - tb_base, kt, kreg, vreg);
       } else {
-        load_kv_tile<BS_CT>(a, bt, head_base, bs, kt, kend, j, g, kreg, vreg);
+        load_kv_tile(a, bt, head_base, bs, kt, kend, j, g, kreg, vreg);
       }
       consume(kt, kreg, vreg);
     }
@@ -622,10 +620,6 @@ int choose_key_split(int64_t tiles) {
 // prompts 3.5 % faster.)
 constexpr int64_t kTwoTileMinTiles = 8192;
 
-// The sequence order applies to one-wave launches only: there, dealing the sequences' tiles
-// longest first (each XCD's share of the heavy sequences, then the rounds' mix) ran 3-16 %
-// faster on six draws of 32 prompts U[256,1024]. Key-split launches hold every workgroup at
-// once and keep the natural order.
 template <int BS>
 void launch_prefill_wide(const PrefillArgs& a_in, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
   PrefillArgs a = a_in;
@@ -643,7 +637,7 @@ void launch_prefill_wide(const PrefillArgs& a_in, hipStream_t stream, hipEvent_t
 // with less work) those
 //  * whose workgroups are well filled: the query rows at least 0.4 of what the grid holds;
 //  * whose tables have room for 256 keys, to amortise a workgroup's start;
-//  * with 1,280 waves of rows (2.5 workgroups for every 2 a CU holds, at 4 waves).
+//  * with 1,280 waves of rows: 320 workgroups of 4, 1.25 a CU, which holds two.
 // Measured us (12 heads; 16-row kernels -> 128-query workgroups), block size 16: 32 prompts of
 // 256-1,023 rows 214 -> 172, 4 x 750-1,000 73 -> 53, 16 x 225-300 34 -> 29, 64 x 75-100 rows behind 200
 // keys 67 -> 47, 2 x 8,192 1,560 -> 1,026 (201 TFLOP/s); left out: 32 x 96-128 18.5 -> 20.0, 64 x 48-64
@@ -673,6 +667,10 @@ void launch_key_split(const PrefillArgs& a, hipStream_t stream, hipEvent_t start
   launch_prefill_ks<BS_CT, KS>(a, stream, start, stop);
 }
 
+// The sequence order applies to one-wave launches only (and to launch_prefill_wide's): there, dealing
+// the sequences' tiles longest first (each XCD's share of the heavy sequences, then the rounds' mix)
+// ran 3-16 % faster on six draws of 32 prompts U[256,1024]. Key-split launches hold every workgroup at
+// once and keep the natural order.
 template <int BS_CT>
 void launch_prefill(const PrefillArgs& a_in, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
   const int ks = choose_key_split((int64_t)a_in.groups * a_in.qtiles);
@@ -681,7 +679,7 @@ void launch_prefill(const PrefillArgs& a_in, hipStream_t stream, hipEvent_t star
   switch (ks) {
     case 1:
       if (BS_CT > 0 && (int64_t)a.num_heads * ((a.num_q_rows + kTile - 1) / kTile) >= kTwoTileMinTiles) {
-        // More tiles than the key split pays for, and many rows: with block size 16 each wave
+        // More tiles than the key split pays for, and many rows: with block size 8, 16 or 32 each wave
         // takes two consecutive query tiles, so every key tile's loads feed both and the wave has
         // two independent softmax chains (per launch: 32 prompts U[256,1024] 248 -> 233 us,
         // 64 prompts x 300 138.6 -> 114.9; 15 prompts U[16,256], 1,530 row tiles, went

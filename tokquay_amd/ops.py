@@ -607,7 +607,7 @@ def _rows_kernel_takes(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | No
     if torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0:
         return False
     return (w.is_contiguous() and x.stride(1) == 1 and x.stride(0) >= k and x.stride(0) % 4 == 0
-            and x.stride(0) < 1 << 21 and k <= 1 << 21
+            and x.stride(0) < 1 << 21  # and k with it
             and (bias is None or (bias.dim() == 1 and bias.size(0) == n and bias.is_contiguous()))
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)  # fmt: skip
 
