@@ -22,7 +22,8 @@
 // The tiles are pipelined so that the scores of tile t + 1 run beside the softmax of tile t and
 // the staging beside the PV product. A 128-query workgroup alone on a CU takes 1.5 us per tile
 // (0.64 us of it MFMA); two per CU reach 201 TFLOP/s of fp32 products (2 x 8,192 rows), which is the
-// rate a large bf16 library product reaches here, a sixth each. Three per CU (168 VGPRs) spill and
+// rate a large bf16 library product reaches here, a sixth each (MFMA busy for 66 % of the cycles at 1.4 GHz: power
+// bound; 44 % at 1.8 GHz for 32 prompts of 256-1,023 rows). Three per CU (168 VGPRs) spill and
 // ran 10 % slower.
 //
 // The softmax is the 16-row kernels' (log2 units, lazy maximum). Queries whose result is not finite are
