@@ -198,8 +198,7 @@ def test_parts_of_k_take_any_bias(gelu):
 
 def test_rule():
     """Few tiles, K not in whole steps: the library; many, or long K to split over the CUs: tq_linear."""
-    assert ops.uses_rows_kernel(96, 768, 3072) and not ops.uses_rows_kernel(95, 768, 3072)
-    assert ops.uses_rows_kernel(320, 512, 3072) and not ops.uses_rows_kernel(319, 512, 3072)
+    assert ops.uses_rows_kernel(320, 768, 3072) and not ops.uses_rows_kernel(319, 768, 3072)
     assert not ops.uses_rows_kernel(640, 768, 768) and not ops.uses_rows_kernel(640, 766, 3072)
     assert not ops.uses_rows_kernel(1536, 768, 3072)  # 144 tiles: neither enough nor few enough for two parts
     assert _lib.lib().tq_linear_workspace_size(1536, 768, 3072) == 0
@@ -275,27 +274,43 @@ def test_tracers_and_modes_see_torch_products(rows):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows", [1, 7, 16, 17, 95, 96, 100, 320, 321])
+@pytest.mark.parametrize("rows", [1, 7, 16, 17, 100, 128, 129, 320, 321])
 def test_few_rows_and_the_head(rows, monkeypatch):
-    """Few rows: long K on tq_linear from 96, short K on the library, the LM head on the library below 64;
-    the same inside a capture as outside one. All within fp32's bound."""
+    """Few rows: the wide layers on tq_linear, the same inside a capture as outside one, and on the library where
+    a step is chosen by GPU time; the LM head on the library below 64 rows. All within fp32's bound."""
     x, w, b = _inputs(rows, 3072, 768)
-    up, down = torch.nn.Linear(768, 3072).cuda(), torch.nn.Linear(3072, 768).cuda()
-    for p in (*up.parameters(), *down.parameters()):
+    up, down, square = torch.nn.Linear(768, 3072).cuda(), torch.nn.Linear(3072, 768).cuda(), torch.nn.Linear(768, 768).cuda()
+    for p in (*up.parameters(), *down.parameters(), *square.parameters()):
         p.requires_grad_(False)
     up.weight.copy_(w), up.bias.copy_(b)
     _check(ops.linear(x, up), x, w, b)
     _check(ops.linear(x, up, gelu=True), x, w, b, gelu=True)
+    _check(ops.linear(x, square), x, square.weight, square.bias)
     h = torch.nn.functional.gelu(x @ w.t() + b, approximate="tanh")
     _check(ops.linear(h, down), h, down.weight, down.bias)
     wide = (torch.randn(50257, 768, generator=torch.Generator().manual_seed(rows)) * 0.02).cuda()
+    _check(ops.lm_head(x, wide), x, wide, None)
+    takes = lambda t, layer: ops._rows_kernel_takes(t, layer.weight, layer.bias)  # noqa: E731
     for capturing in (False, True):
         monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
-        assert not ops._rows_kernel_takes(x, up.weight, up.bias)
-        assert ops._rows_kernel_takes(h, down.weight, down.bias) == (rows >= 96)
+        assert takes(x, up) == (rows <= 320) and takes(h, down) and takes(x, square) == (rows <= 128)
         assert ops._rows_kernel_takes(x, wide, None) == (rows >= 64)
-    monkeypatch.undo()
-    _check(ops.lm_head(x, wide), x, wide, None)
+        with ops.by_gpu_time():
+            assert not takes(x, up) and takes(h, down) == (rows >= 320) and not takes(x, square)
+            assert ops._rows_kernel_takes(x, wide, None) == (rows >= 64)
+
+
+def test_few_rows_rule():
+    """The cheaper call only where the GPU keeps up with it: not for an LM head's weights, nor where long K is left
+    in few parts."""
+    for m, n, k in ((1, 3072, 768), (128, 768, 768), (320, 768, 3072), (256, 1600, 6400), (128, 768, 3136)):
+        assert ops._saves_host_time(m, n, k)
+        with ops.by_gpu_time():
+            assert not ops._saves_host_time(m, n, k)
+        assert ops._saves_host_time(m, n, k)
+    for m, n, k in ((0, 3072, 768), (8, 32000, 768), (129, 768, 768), (321, 768, 3072), (128, 766, 768), (128, 768, 776),
+                    (128, 768, 3104), (320, 768, 3296), (320, 1600, 6400), (320, 768, 8192)):  # fmt: skip
+        assert not ops._saves_host_time(m, n, k)
 
 
 CAPTURE = """
@@ -319,10 +334,10 @@ print("captured")
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows", [64, 100, 256])
+@pytest.mark.parametrize("rows", [64, 100, 256, 400])
 def test_one_eager_run_prepares_a_capture(rows):
     """In a process that has run nothing else, the MLP's layers are captured after one eager run, and every
-    replay gives the eager call's bits (256 rows: through the transposed weights)."""
+    replay gives the eager call's bits."""
     run = subprocess.run([sys.executable, "-c", CAPTURE.format(rows=rows)], capture_output=True, text=True, timeout=100,
                          cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))  # fmt: skip
     assert run.returncode == 0 and "captured" in run.stdout, run.stderr[-2000:]

@@ -177,13 +177,14 @@ class DecodeGraphs:
         tokens = s.tokens.clone()  # the warm-up runs overwrite what this step's source rows read
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side):  # warm-up launches (same inputs: the K/V writes are idempotent)
+        # Warm-up launches of what is captured (same inputs: the K/V writes are idempotent).
+        with torch.cuda.stream(side), ops.by_gpu_time():
             for _ in range(2):
                 self._forward(rows, ids_only)
                 s.tokens.copy_(tokens)
         torch.cuda.current_stream().wait_stream(side)
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
+        with torch.cuda.graph(graph), ops.by_gpu_time():
             logits = self._forward(rows, ids_only)
         self.graphs[(rows, ids_only)] = (graph, logits)
 

@@ -16,8 +16,10 @@ Shapes (fp32 unless noted; ``H`` heads of ``D = 64`` dims):
 
 from __future__ import annotations
 
+import contextlib
 import functools
 import math
+import threading
 
 import torch
 from torch.utils._device import DeviceContext
@@ -539,22 +541,45 @@ def uses_nn_layout(rows: int, out_features: int, in_features: int, gelu: bool) -
 # [640, 2304, 768] 180 tiles 25.6 -> 19.2; [2048, 768, 768] 192 tiles 26.1 -> 19.9; [2048, 768, 3072] 192 tiles
 # 78.8 -> 66.4; [65, 50257, 768] 786 tiles 69.8 -> 52.7; [8192, 3072, 768] 3,072 tiles 280 -> 191.
 # With fewer tiles, long K is worth splitting over the idle CUs (tq_linear does, and sums the parts in a
-# second launch) where the parts give as many CUs work as that: [384 / 640 / 768 / 1280, 768, 3072] 28.2 / 30.7 /
-# 41.3 / 54.6 -> 21.5 / 27.9 / 33.2 / 46.0, [512, 1024, 4096] 37.7 -> 33.5, [512, 1600, 6400] 96 -> 73, but [320,
-# 1600, 6400] (150 parts in all) 54 -> 70, [640, 768, 3136] (120) 31 -> 37 and [320, 768, 3104] (K of 97 steps:
-# no split) 28 -> 56. From 96 rows on where the output is 768 wide or more: [96 / 128 / 192 / 256, 768, 3072] 16.1 /
-# 16.1 / 18.1 / 18.4 -> 14.2 / 15.6 / 16.8 / 18.0, [96, 1600, 6400] 37 -> 24, [160, 1024, 4096] 23.2 -> 20.6; it gives a
-# little between ([160 / 320, 768, 3072] 15.6 / 18.0 -> 17.1 / 18.8), for a call that takes the host 9 us and not 19. Below
-# 96 rows the library is faster ([65, 768, 3072] 10.7 -> 13.7), and so it is for narrow outputs of few rows ([128 / 256,
-# 512, 3072] 9.7 / 14.2 -> 13.8 / 15.5; at 320 17.5 -> 16.7). Short K stays with the library: [640, 768, 768]
-# 10.2 -> 15.2.
+# second launch) from 320 rows on, where the parts give as many CUs work as that: [384 / 640 / 768 / 1280, 768,
+# 3072] 28.2 / 30.7 / 41.3 / 54.6 -> 21.5 / 27.9 / 33.2 / 46.0, [512, 1024, 4096] 37.7 -> 33.5, [512, 1600, 6400] 96 -> 73,
+# but [320, 1600, 6400] (150 parts in all) 54 -> 70, [640, 768, 3136] (120) 31 -> 37 and [320, 768, 3104] (K of 97
+# steps: no split) 28 -> 56. Fewer rows and short K stay with the library: [256 / 300, 768, 3072] 18.9 / 19.4 -> 18.6 /
+# 20.2, [300, 1600, 6400] 59 -> 76, [640, 768, 768] 10.2 -> 15.2.
 # Fewer than 64 rows leave the 128-row tiles mostly padding, however many they are: the LM head [rows, 50257,
 # 768] 8 / 32 / 48 / 64 / 128 rows 33 / 37 / 45 / 67 / 104 -> 53 / 52 / 55 / 57 / 70.
 ROWS_KERNEL_MIN_TILES = 160
 ROWS_KERNEL_MIN_ROWS = 64
-SPLIT_MIN_K = 3072
-SPLIT_MIN_ROWS, SPLIT_MIN_WIDTH, SPLIT_NARROW_MIN_ROWS = 96, 768, 320
+SPLIT_MIN_ROWS, SPLIT_MIN_K = 320, 3072
+# Up to some rows an eager step is bound by the host: the library call takes it about 19 us, tq_linear
+# about 9, for about the same GPU time in the wide layers ([64-256, 3072, 768] 10-16 -> 12-19 us,
+# [64-256, 768, 3072] 11-18 -> 13-18): the MLP over 256 rows 39 -> 34 us a call, over 64 45 -> 27. The
+# narrower ones ([2304, 768] 10-14 -> 11-14 us, [768, 768] 7 -> 10 at 64-128 rows) follow up to 128 rows; at
+# 256 (14.5 -> 16, 7 -> 12) the layer with its attention is bound by the GPU: 182.0 -> 182.9 us.
+# The choice is by sizes only, so that an eager call and a captured one of the same sizes run the same kernel and
+# one eager run loads and allocates what a capture needs (the library's handle cannot be made inside one).
+# Replays cost the host nothing: DecodeGraphs warms up and captures its steps by GPU time, from the library where
+# it is faster, and rounds differently from eager steps of the same rows.
+FEW_ROWS, FEW_ROWS_WIDTH = 320, 3072
+FEW_ROWS_NARROW, FEW_ROWS_NARROW_WIDTH = 128, 768
+FEW_ROWS_MAX_WEIGHTS = 1600 * 6400  # [16-128, 1600, 6400] 20-38 -> 22-27 us; the LM head (above) is bound by the GPU
+# K a workgroup walks by itself: past this the GPU's time is the longer one. [128, 768, 3104] (no split) 19 -> 56 us a
+# call, [320, 1600, 6400] (3,200) 57 -> 68, [320, 768, 8192] (2,048) 43 -> 46, but [256, 1600, 6400] (1,280) 53 -> 40.
+FEW_ROWS_MAX_PART = 1280
 _TENSORS = (torch.Tensor, torch.nn.Parameter)
+_choice = threading.local()
+
+
+@contextlib.contextmanager
+def by_gpu_time():
+    """The calling thread's linears inside are chosen by their GPU time alone: for a step that is captured
+    once and replayed. Both the runs that prepare the capture and the capture itself belong inside."""
+    before = getattr(_choice, "gpu_time", False)
+    _choice.gpu_time = True
+    try:
+        yield
+    finally:
+        _choice.gpu_time = before
 
 
 @functools.lru_cache(maxsize=1024)
@@ -565,16 +590,24 @@ def _split_parts(rows: int, out_features: int, in_features: int) -> int:
 
 
 def uses_rows_kernel(rows: int, out_features: int, in_features: int) -> bool:
-    """Whether a linear layer of these sizes runs on ``tq_linear`` (else on the library GEMM), eager and
-    under capture alike."""
+    """Whether a linear layer of these sizes takes the GPU less time on ``tq_linear`` than on the library."""
     if rows < ROWS_KERNEL_MIN_ROWS or in_features % 32 or in_features == 0:
         return False
     tiles = ((rows + 127) >> 7) * ((out_features + 63) >> 6)
     if tiles >= ROWS_KERNEL_MIN_TILES:
         return True
-    if in_features < SPLIT_MIN_K or rows < (SPLIT_MIN_ROWS if out_features >= SPLIT_MIN_WIDTH else SPLIT_NARROW_MIN_ROWS):
+    if in_features < SPLIT_MIN_K or rows < SPLIT_MIN_ROWS:
         return False
     return _split_parts(rows, out_features, in_features) * tiles >= ROWS_KERNEL_MIN_TILES
+
+
+def _saves_host_time(rows: int, out_features: int, in_features: int) -> bool:
+    """Whether a linear layer of few rows runs on ``tq_linear`` for its cheaper call."""
+    if getattr(_choice, "gpu_time", False) or not 0 < rows <= FEW_ROWS or in_features % 32 or out_features % 4:
+        return False
+    wide = FEW_ROWS_WIDTH if rows > FEW_ROWS_NARROW else FEW_ROWS_NARROW_WIDTH
+    return (max(out_features, in_features) >= wide and out_features * in_features <= FEW_ROWS_MAX_WEIGHTS
+            and in_features <= FEW_ROWS_MAX_PART * _split_parts(rows, out_features, in_features))  # fmt: skip
 
 
 def _recorded() -> bool:
@@ -588,16 +621,16 @@ def _recorded() -> bool:
 
 
 def _rows_kernel_takes(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None) -> bool:
-    """Whether ``x @ w.T + bias`` goes to ``tq_linear``: by its sizes (``uses_rows_kernel``), for plain
-    float32 tensors on one HIP device in the layout it reads, and if nothing must see torch's own
-    product (a gradient, a functorch transform, forward-mode AD, a tensor subclass, autocast, a tracer
-    or mode)."""
+    """Whether ``x @ w.T + bias`` goes to ``tq_linear``: by its sizes (``uses_rows_kernel``,
+    ``_saves_host_time``), for plain float32 tensors on one HIP device in the layout it reads, and if
+    nothing must see torch's own product (a gradient, a functorch transform, forward-mode AD, a tensor
+    subclass, autocast, a tracer or mode)."""
     if _recorded() or torch.is_autocast_enabled("cuda"):  # torch's products return the autocast type
         return False
     n, k = w.shape
     if x.dim() != 2 or x.size(1) != k:
         return False
-    if not uses_rows_kernel(x.size(0), n, k):
+    if not uses_rows_kernel(x.size(0), n, k) and not _saves_host_time(x.size(0), n, k):
         return False
     ts = (x, w) if bias is None else (x, w, bias)
     if any(type(t) not in _TENSORS or t.dtype != torch.float32 or t.device != x.device for t in ts):
@@ -628,7 +661,7 @@ def lm_head(h: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 def linear(x: torch.Tensor, layer: torch.nn.Linear, gelu: bool = False) -> torch.Tensor:
     """``x @ layer.weight.T + layer.bias`` (then the tanh GELU when ``gelu``): ``tq_linear`` over many
-    rows (``uses_rows_kernel``), else hipBLASLt in the weight layout ``GEMM_NN_SHAPES`` names for
+    rows and for cheaper calls of few (``_rows_kernel_takes``), else hipBLASLt in the weight layout ``GEMM_NN_SHAPES`` names for
     this shape. On the CPU: torch's ``F.linear`` and the tanh GELU."""
     weight, bias = layer.weight, layer.bias  # each a Module lookup: once
     if not x.is_cuda:
