@@ -322,7 +322,7 @@ def prefill_batch(seed: int = 32, reps: int = 3) -> dict:
     """The prefill kernel on a large launch, as the engine's prefill steps run it: one prefill step of
     32 prompts of U[256,1024] random tokens (block size 16) through the model, every layer's
     tq_paged_prefill launch timed by the events it records; causal-exact flops over the launch time
-    against the fp32 MFMA peak. The step runs reps times from the same state (its cache writes are the
+    against a sixth of the bf16 MFMA peak. The step runs reps times from the same state (its cache writes are the
     same each time); the median per layer over all runs."""
     import torch
 
