@@ -211,6 +211,7 @@ def test_rule():
         assert not ops.uses_rows_kernel(m, n, k)
     assert ops.uses_rows_kernel(512, 1600, 6400) and ops.uses_rows_kernel(320, 768, 3136)
     assert ops.uses_rows_kernel(65, 50257, 768) and not ops.uses_rows_kernel(63, 50257, 768)
+    assert not ops.uses_rows_kernel(400, 0, 3072)
     assert not ops.uses_rows_kernel(8192, 3072, 776) and not ops.uses_rows_kernel(8192, 3072, 0)
 
 
@@ -308,9 +309,22 @@ def test_few_rows_rule():
         with ops.by_gpu_time():
             assert not ops._saves_host_time(m, n, k)
         assert ops._saves_host_time(m, n, k)
-    for m, n, k in ((0, 3072, 768), (8, 32000, 768), (129, 768, 768), (321, 768, 3072), (128, 766, 768), (128, 768, 776),
+    for m, n, k in ((0, 3072, 768), (100, 3072, 0), (100, 0, 3072), (8, 32000, 768), (129, 768, 768), (321, 768, 3072), (128, 766, 768), (128, 768, 776),
                     (128, 768, 3104), (320, 768, 3296), (320, 1600, 6400), (320, 768, 8192)):  # fmt: skip
         assert not ops._saves_host_time(m, n, k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [0, 1, 100, 400])
+@pytest.mark.parametrize("k,n", [(0, 768), (0, 3072), (768, 0), (3072, 0), (768, 3072)])
+def test_empty_layers_and_batches(rows, k, n):
+    """No rows, no outputs, or an empty sum (the bias): torch's result."""
+    layer = torch.nn.Linear(768, 3072).cuda().requires_grad_(False)
+    layer.weight, layer.bias = (torch.nn.Parameter(torch.randn(s, device="cuda"), False) for s in ((n, k), (n,)))
+    x = torch.randn(rows, k, device="cuda")
+    want = torch.addmm(layer.bias, x, layer.weight.t())
+    torch.testing.assert_close(ops.linear(x, layer), want, rtol=1e-4, atol=1e-3)
+    torch.testing.assert_close(ops.lm_head(x, layer.weight), x @ layer.weight.T, rtol=1e-4, atol=1e-3)
 
 
 CAPTURE = """

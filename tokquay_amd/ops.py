@@ -503,7 +503,8 @@ def embed_rows(ids: torch.Tensor, positions: torch.Tensor, wte: torch.Tensor, wp
 # [768] -> [3072]) 16.7 -> 13.7 us. At 224 or 320 rows, and for the [3072] -> [768] projection at
 # any row count, the weight as stored ("TN") is as fast or faster. The choice is this fixed table,
 # not a measurement at run time, so that every process computes every shape the same way (the two
-# layouts may round differently) and no live step pays for a probe.
+# layouts may round differently, and tq_linear, on which eager steps of 256 rows run where DecodeGraphs
+# captures these, differently again) and no live step pays for a probe.
 GEMM_NN_SHAPES: frozenset[tuple[int, int, int, bool]] = frozenset({
     (256, 2304, 768, False),  # c_attn at the 256-row decode bucket
     (256, 3072, 768, True),  # c_fc + GELU at the 256-row decode bucket
@@ -591,7 +592,7 @@ def _split_parts(rows: int, out_features: int, in_features: int) -> int:
 
 def uses_rows_kernel(rows: int, out_features: int, in_features: int) -> bool:
     """Whether a linear layer of these sizes takes the GPU less time on ``tq_linear`` than on the library."""
-    if rows < ROWS_KERNEL_MIN_ROWS or in_features % 32 or in_features == 0:
+    if rows < ROWS_KERNEL_MIN_ROWS or in_features % 32 or in_features == 0 or out_features == 0:
         return False
     tiles = ((rows + 127) >> 7) * ((out_features + 63) >> 6)
     if tiles >= ROWS_KERNEL_MIN_TILES:
@@ -603,7 +604,8 @@ def uses_rows_kernel(rows: int, out_features: int, in_features: int) -> bool:
 
 def _saves_host_time(rows: int, out_features: int, in_features: int) -> bool:
     """Whether a linear layer of few rows runs on ``tq_linear`` for its cheaper call."""
-    if getattr(_choice, "gpu_time", False) or not 0 < rows <= FEW_ROWS or in_features % 32 or out_features % 4:
+    if getattr(_choice, "gpu_time", False) or not 0 < rows <= FEW_ROWS or in_features % 32 or out_features % 4 \
+            or in_features == 0 or out_features == 0:
         return False
     wide = FEW_ROWS_WIDTH if rows > FEW_ROWS_NARROW else FEW_ROWS_NARROW_WIDTH
     return (max(out_features, in_features) >= wide and out_features * in_features <= FEW_ROWS_MAX_WEIGHTS
