@@ -327,6 +327,21 @@ def test_empty_layers_and_batches(rows, k, n):
     torch.testing.assert_close(ops.lm_head(x, layer.weight), x @ layer.weight.T, rtol=1e-4, atol=1e-3)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [100, 800])
+def test_tensors_without_strided_storage(rows):
+    """Sparse rows or weights and zero tensors: torch's result."""
+    layer = torch.nn.Linear(768, 3072).cuda().requires_grad_(False)
+    x = torch.randn(rows, 768, device="cuda")
+    want = torch.addmm(layer.bias, x, layer.weight.t())
+    for t in (x.to_sparse(), x.to_sparse_csr()):
+        torch.testing.assert_close(ops.linear(t, layer), want, rtol=1e-4, atol=1e-4)
+    zeros = torch._efficientzerotensor((rows, 768), device="cuda")
+    torch.testing.assert_close(ops.linear(zeros, layer), layer.bias.expand(rows, -1))
+    layer.weight = torch.nn.Parameter(layer.weight.to_sparse_csr(), False)
+    torch.testing.assert_close(ops.linear(x, layer), want, rtol=1e-4, atol=1e-4)
+
+
 CAPTURE = """
 import torch
 from tokquay_amd import ops

@@ -558,7 +558,8 @@ SPLIT_MIN_ROWS, SPLIT_MIN_K = 320, 3072
 # narrower ones ([2304, 768] 10-14 -> 11-14 us, [768, 768] 7 -> 10 at 64-128 rows) follow up to 128 rows; at
 # 256 (14.5 -> 16, 7 -> 12) the layer with its attention is bound by the GPU: 182.0 -> 182.9 us.
 # The choice is by sizes only, so that an eager call and a captured one of the same sizes run the same kernel and
-# one eager run loads and allocates what a capture needs (the library's handle cannot be made inside one).
+# one eager run loads and allocates what a capture needs (the library's handle cannot be made inside one); a
+# caller's own replays pay the GPU times above.
 # Replays cost the host nothing: DecodeGraphs warms up and captures its steps by GPU time, from the library where
 # it is faster, and rounds differently from eager steps of the same rows.
 FEW_ROWS, FEW_ROWS_WIDTH = 320, 3072
@@ -635,7 +636,8 @@ def _rows_kernel_takes(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | No
     if not uses_rows_kernel(x.size(0), n, k) and not _saves_host_time(x.size(0), n, k):
         return False
     ts = (x, w) if bias is None else (x, w, bias)
-    if any(type(t) not in _TENSORS or t.dtype != torch.float32 or t.device != x.device for t in ts):
+    if any(type(t) not in _TENSORS or t.dtype != torch.float32 or t.device != x.device or t.layout != torch.strided
+           or t._is_zerotensor() for t in ts):  # fmt: skip
         return False
     if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
         return False
